@@ -385,14 +385,14 @@ struct PrefillLaunch {
     int32_t kernel;     // PREFILL_KERNEL_*: which form runs where several exist
     int32_t item_rows;  // query rows per work item of `work` (64, or PREFILL_WIDE_ROWS)
 };
-// Query rows per work item of the wide list (the default kernel at hd 128).
+// Query rows per work item of the wide list (the default kernel past hd 64).
 constexpr int32_t PREFILL_WIDE_ROWS = 128;
 // Whether a launch of this kernel / head_dim takes the wide work list.
 bool prefill_uses_wide_items(int32_t kernel, int32_t head_dim);
 // Whether this kernel / head_dim has the appending form (PrefillLaunch::k_new)
 // for a batch whose largest position is max_pos (its table rows fit in LDS).
 bool prefill_appends_in_launch(int32_t kernel, int32_t head_dim, int32_t max_pos, int64_t page_stride);
-constexpr int32_t PREFILL_KERNEL_DEFAULT = 0;   // bf16 matrix cores at fp32 accuracy (hd <= 128)
+constexpr int32_t PREFILL_KERNEL_DEFAULT = 0;   // bf16 matrix cores at fp32 accuracy
 constexpr int32_t PREFILL_KERNEL_VALU = 1;      // fp32 VALU FMAs
 constexpr int32_t PREFILL_KERNEL_MFMA_F32 = 2;  // fp32 matrix cores (v_mfma_f32_16x16x4_f32)
 // Query rows per prefill work item.

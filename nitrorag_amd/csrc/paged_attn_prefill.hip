@@ -6,13 +6,12 @@
 // earlier chunks and the chunk's own rows, already scattered into the pool).
 //
 // Three kernels, all at fp32 accuracy:
-//  - paged_attn_prefill_x3_kernel (hd 32/64/128, the default): the bf16
-//    matrix cores on exact three-part bf16 splits of Q, K, V and P (its
-//    comment below);
+//  - paged_attn_prefill_x3_kernel (the default, every head size): the bf16
+//    matrix cores on exact bf16 splits of Q, K, V and P (its comment below);
 //  - paged_attn_prefill_mfma_kernel (NITRO_PREFILL_KERNEL=mfma32): the fp32
 //    matrix cores;
-//  - paged_attn_prefill_kernel (hd 256, or NITRO_PREFILL_KERNEL=valu): fp32
-//    VALU FMAs.
+//  - paged_attn_prefill_kernel (NITRO_PREFILL_KERNEL=valu, and mfma32 at head
+//    sizes other than 32, 64, 128): fp32 VALU FMAs.
 //
 // paged_attn_prefill_mfma_kernel<hd, QT, KSPLIT, BNM> runs both matrix
 // products on v_mfma_f32_16x16x4_f32 (fp32 inputs, fp32 accumulate):
@@ -41,7 +40,7 @@
 //  - Key groups hand (m, l, O) to key group 0 through LDS at the end.
 //
 // paged_attn_prefill_kernel<HDP, FULL> (any head size that is a multiple of
-// 4 up to 256; used for hd 256 and sizes other than 32/64/128) is the VALU form:
+// 4 up to 256) is the VALU form:
 //  - A work item is up to BM=64 query rows of one chunk; grid = (work items,
 //    heads).  The host sorts work items by key count, longest first.
 //  - 256 threads: 4 lanes per query row, each lane holding hd/4 of q and of
@@ -574,18 +573,27 @@ __global__ __launch_bounds__(64 * QT * KSPLIT) void paged_attn_prefill_mfma_kern
     }
 }
 
-// paged_attn_prefill_x3_kernel<hd, KSPLIT, BNM>: the MFMA kernel's work
-// split and softmax with both products on the bf16 matrix cores at fp32
-// accuracy.  Q and K are each split into three bf16 parts (hi, mid, lo;
-// exact, 24 significant bits in all), and S = K Q^T takes the six part
-// products whose order is at most 2 (hi.hi, hi.mid, mid.hi, hi.lo, mid.mid,
-// lo.hi; the dropped ones are below 2^-24 of the total): an error in S moves
-// every weight exponentially, so S keeps fp32 accuracy.  V and the
-// probabilities P are split into two (hi, mid: 16 significant bits, the rest
-// below 2^-16 of each value), and O takes the four products V.P (mid.mid,
-// mid.hi, hi.mid, hi.hi): O is a weighted average of V, so relative errors
-// of at most 2^-16 in V and P move it by at most about 3e-5 of the values'
-// size.  All accumulate in fp32 by v_mfma_f32_16x16x32_bf16, smallest first:
+// paged_attn_prefill_x3_kernel<HDL, HD, FULL, VP, QT, KSPLIT, BNM, APPEND>: the
+// MFMA kernel's work split and softmax with both products on the bf16 matrix
+// cores at fp32 accuracy.  Q and K are each split into three bf16 parts (hi,
+// mid, lo; exact, 24 significant bits in all), and S = K Q^T takes the six
+// part products whose order is at most 2 (hi.hi, hi.mid, mid.hi, hi.lo,
+// mid.mid, lo.hi; the dropped ones are below 2^-24 of the total): an error in
+// S moves every weight exponentially, so S keeps fp32 accuracy.  V and the
+// probabilities P are split into VP parts:
+//  - VP 2 (head sizes 32, 64, 128): hi, mid, 16 significant bits, the rest
+//    below 2^-16 of each value, and O takes the four products V.P (mid.mid,
+//    mid.hi, hi.mid, hi.hi): O is a weighted average of V, so relative errors
+//    of at most 2^-16 in V and P move it by at most about 3e-5 of the values'
+//    size;
+//  - VP 3 (every other head size): all 24 bits and the six products of order
+//    at most 2, fp32 accuracy throughout.  S is held there as two sums, hi.hi
+//    and the five small products, added once at the end of the row: error
+//    against 64 bits 1.9e-7 (2-norm) on 6 prompts of 50-700 tokens at 16 x 96,
+//    2.3e-7 as one sum, 2.6e-7 with fp32 VALU sums (0.87e-7 / 1.2e-7 / 1.0e-7
+//    at 17 tokens).  Holding O's small products apart too gave 1.4e-7 for 7%
+//    more time.
+// All accumulate in fp32 by v_mfma_f32_16x16x32_bf16, smallest first:
 //  - S^T = K Q^T per 16-key block and 32 d: lane l supplies K[key l%16] and
 //    Q[query l%16] at d = 32c + 8*(l/16) .. +8, so the accumulator leaves lane
 //    l holding S[query l%16][keys 4g..4g+3] (g = l/16) as before;
@@ -593,11 +601,20 @@ __global__ __launch_bounds__(64 * QT * KSPLIT) void paged_attn_prefill_mfma_kern
 //    is its own probabilities of the two blocks (keys 4g..4g+3 of each), and
 //    its A operand V^T[d = 16n + l%16] at the same 8 keys, read from a
 //    transposed V tile.
+// Head sizes: the products run at HD columns (32, 64, 96, 128 or 256, the head
+// size rounded up; FULL: it is HD), and a row's load slots are dealt to the
+// threads HDL (HD rounded up to a power of two) columns apart, so that a
+// thread's column is the same in every load.  Columns between the head size
+// and HD are staged as zero.  These sizes ran on the VALU kernel before, which
+// is bound by its FMAs and LDS reads: 6 prompts of 50-700 tokens at 16 x 96
+// 445 -> 70 us per layer with the append, 16 x 256 900 -> 160, 32 x 80 450 ->
+// 125, 12 x 48 135 -> 50; one 4000-token prompt at 16 x 96 2.43 -> 0.33 ms;
+// one token the same.
 // A workgroup serves one work item of 16*QT query rows (QT = 8: 128 rows,
 // the wide work list, so each staged tile serves twice the queries) with QT
 // query sub-tiles x KSPLIT key groups of waves.
 // K and V are split once, when a tile is staged: three bf16 planes of K and
-// two of V in LDS, K as [key][d] and V as [d][key].  K is loaded a float4 of one key row
+// VP of V in LDS, K as [key][d] and V as [d][key].  K is loaded a float4 of one key row
 // per thread; V one d of four consecutive keys per thread (a wave's lanes
 // cover consecutive d of a row, so the loads coalesce), which becomes one
 // 8-byte store per plane into the transposed tile.
@@ -611,15 +628,17 @@ __global__ __launch_bounds__(64 * QT * KSPLIT) void paged_attn_prefill_mfma_kern
 // at position 0), every key new.  APPEND 2: chunks after cached keys; a key
 // below its chunk's start is read from the pool, the others from the new
 // rows, chosen per key (a tile may hold both).
-template <int HD, int QT, int KSPLIT, int BNM, int APPEND>
+template <int HDL, int HD, bool FULL, int VP, int QT, int KSPLIT, int BNM, int APPEND>
 // Up to hd 64 two workgroups share a CU (LDS), which takes at most 128
-// VGPRs (4 waves per SIMD); hd 128 runs one workgroup per CU.
+// VGPRs (4 waves per SIMD); larger heads run one workgroup per CU.
 __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn_prefill_x3_kernel(PrefillLaunch a) {
     constexpr int NT = 64 * QT * KSPLIT;
     constexpr int KB = BNM / 16;               // 16-key blocks per tile
     constexpr int NBW = KB / KSPLIT;           // 16-key blocks per wave per tile
     static_assert(KB % KSPLIT == 0 && NBW % 2 == 0, "a wave's blocks pair up into 32-key products");
-    constexpr int F4 = HD / 4;                 // float4 per K/V row
+    static_assert(HD % 32 == 0 && HDL >= HD && (HDL & (HDL - 1)) == 0, "head size");
+    static_assert(VP == 2 || VP == 3, "parts of V and P");
+    constexpr int F4 = HDL / 4;                // float4 slots per K/V row
     constexpr int NC = HD / 32;                // 32-d chunks of S
     constexpr int NB = HD / 16;                // 16-column blocks of the output
     // K plane row (bf16; 16-byte aligned rows).  HD + 16 measured 64% fewer
@@ -630,18 +649,27 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
     constexpr int KST = HD + 16;
     constexpr int VST = BNM + 4;               // V^T plane row (bf16; 8-byte aligned rows, stores spread over banks)
     constexpr int LOADS = BNM * F4 / NT;       // K float4 per thread per tile
-    constexpr int VSLOTS = BNM * HD / (4 * NT);  // V (d, 4-key group) slots per thread per tile
-    static_assert(LOADS >= 1 && BNM * F4 % NT == 0 && VSLOTS >= 1 && BNM * HD % (4 * NT) == 0, "tile shape");
+    constexpr int VSLOTS = BNM * HDL / (4 * NT);  // V (d, 4-key group) slots per thread per tile
+    static_assert(LOADS >= 1 && BNM * F4 % NT == 0 && VSLOTS >= 1 && BNM * HDL % (4 * NT) == 0, "tile shape");
     constexpr int KPLANE = BNM * KST, VPLANE = HD * VST;
-    static_assert((KSPLIT - 1) * QT * 16 * HD * 4 <= (3 * KPLANE + 2 * VPLANE) * 2, "partials fit the tile planes");
-    // K in three bf16 planes, V^T in two
-    __shared__ __attribute__((aligned(16))) uint16_t kv_lds[3 * KPLANE + 2 * VPLANE];
+    static_assert((KSPLIT - 1) * QT * 16 * HD * 4 <= (3 * KPLANE + VP * VPLANE) * 2, "partials fit the tile planes");
+    // K in three bf16 planes, V^T in VP
+    __shared__ __attribute__((aligned(16))) uint16_t kv_lds[3 * KPLANE + VP * VPLANE];
     uint16_t* const k_lds = kv_lds;
     uint16_t* const v_lds = kv_lds + 3 * KPLANE;
     __shared__ int32_t s_table[TABLE_LDS];
     __shared__ float s_ml[KSPLIT > 1 ? QT * (KSPLIT - 1) * 16 * 2 : 1];
     __shared__ int32_t s_wave_bad[NT / 64];
 
+    const int hd = FULL ? HD : a.head_dim;
+    // This thread's column of a row in its K loads (a float4) and V loads: the
+    // same in every load (NT is a multiple of a row's slots).  A slot past the
+    // head reads column 0 and is staged as zero.
+    static_assert(NT % F4 == 0 && NT % HDL == 0, "a thread's column is the same in every load");
+    const int kslot = (int)(threadIdx.x % F4) * 4, vslot = (int)(threadIdx.x % HDL);
+    const bool kcol_ok = (FULL && HDL == HD) || kslot < hd, vcol_ok = (FULL && HDL == HD) || vslot < hd;
+    const bool kreal = FULL || kslot < hd, vreal = FULL || vslot < hd;  // (slots past HD are not staged)
+    const int kcol = kcol_ok ? kslot : 0, vcol = vcol_ok ? vslot : 0;
     const int h = blockIdx.x % a.n_heads;
     const int item = blockIdx.x / a.n_heads;
     const int seq = a.work[2 * item];
@@ -662,7 +690,7 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
     const int wave_first = start + q0 + min(qs * 16, qcount - 1);
     const int32_t* trow = a.tables + (size_t)seq * a.max_pages;
     const int n_tiles = last_pos / BNM + 1;
-    const size_t dim = (size_t)a.n_heads * HD;
+    const size_t dim = (size_t)a.n_heads * hd;
     const size_t qrow = (size_t)(a.row_off[seq] + q0 + min(row, qcount - 1));
 
     // This lane's query at d = 32c + 8g .. +8, loaded before the table so the
@@ -671,9 +699,10 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
     float4 qraw[NC][2];
 #pragma unroll
     for (int c = 0; c < NC; c++) {
-        const float4* src = reinterpret_cast<const float4*>(a.q + qrow * dim + (size_t)h * HD + 32 * c + 8 * g);
-        qraw[c][0] = src[0];
-        qraw[c][1] = src[1];
+        const float4* src = reinterpret_cast<const float4*>(a.q + qrow * dim + (size_t)h * hd + 32 * c + 8 * g);
+        const float4 none = make_float4(0.f, 0.f, 0.f, 0.f);
+        qraw[c][0] = FULL || 32 * c + 8 * g < hd ? src[0] : none;
+        qraw[c][1] = FULL || 32 * c + 8 * g + 4 < hd ? src[1] : none;
     }
 
     f32x4 acc[NB];
@@ -681,8 +710,8 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
     for (int n = 0; n < NB; n++) acc[n] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m = -INFINITY, lsum = 0.0f;
 
-    const float* kbase = a.k_pool + a.layer_off + (size_t)kv_h * HD;
-    const float* vbase = a.v_pool + a.layer_off + (size_t)kv_h * HD;
+    const float* kbase = a.k_pool + a.layer_off + (size_t)kv_h * hd;
+    const float* vbase = a.v_pool + a.layer_off + (size_t)kv_h * hd;
     float4 kreg[LOADS];
     float vreg[VSLOTS][4];
     // Fetch: a tile's page ids are all looked up first, then every K/V load
@@ -703,50 +732,52 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
             kpage[i] = page_of(min(tile * BNM + (int)(threadIdx.x + i * NT) / F4, last_pos));
 #pragma unroll
         for (int i = 0; i < VSLOTS; i++)
-            vpage[i] = page_of(min(tile * BNM + 4 * ((int)(threadIdx.x + i * NT) / HD), last_pos));
+            vpage[i] = page_of(min(tile * BNM + 4 * ((int)(threadIdx.x + i * NT) / HDL), last_pos));
         kmask = vmask = 0;
 #pragma unroll
         for (int i = 0; i < LOADS; i++) {
             const int f = threadIdx.x + i * NT;
-            const int r = f / F4, col = f % F4;
+            const int r = f / F4;
             const int key = tile * BNM + r;
             const bool in = key <= last_pos;
             const bool ok = in && (unsigned)kpage[i] < (unsigned)a.num_pages;
-            if (in && !ok && col == 0) atomicAdd(a.bad_pages, 1);  // once per key (V reads the same page)
-            kmask |= (uint32_t)ok << i;
+            if (in && !ok && kslot == 0) atomicAdd(a.bad_pages, 1);  // once per key (V reads the same page)
+            kmask |= (uint32_t)(ok && kreal) << i;
             const size_t off = ok ? (size_t)kpage[i] * a.page_stride + (size_t)(key & 15) * a.kv_dim : 0;
-            kreg[i] = reinterpret_cast<const float4*>(kbase + off)[col];
+            kreg[i] = *reinterpret_cast<const float4*>(kbase + off + kcol);
         }
 #pragma unroll
         for (int i = 0; i < VSLOTS; i++) {
             const int sl = threadIdx.x + i * NT;
-            const int d = sl % HD, key0 = tile * BNM + 4 * (sl / HD);  // 4 keys, one page
+            const int key0 = tile * BNM + 4 * (sl / HDL);  // 4 keys, one page
             const bool ok = key0 <= last_pos && (unsigned)vpage[i] < (unsigned)a.num_pages;
-            const float* vp = vbase + (ok ? (size_t)vpage[i] * a.page_stride : 0) + (size_t)(key0 & 15) * a.kv_dim + d;
+            const float* vp = vbase + (ok ? (size_t)vpage[i] * a.page_stride : 0) + (size_t)(key0 & 15) * a.kv_dim + vcol;
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 vreg[i][e] = vp[(size_t)e * a.kv_dim];
-                vmask |= (uint32_t)(ok && key0 + e <= last_pos) << (4 * i + e);
+                vmask |= (uint32_t)(ok && vreal && key0 + e <= last_pos) << (4 * i + e);
             }
         }
     };
     // With the whole table in LDS, a thread's loads differ from tile to tile
     // only in their page ids: its K loads read row (tid / F4) % 16 of a page at
-    // column tid % F4, its V slots rows 4 * (tid / HD) % 16 .. +3 at column
-    // tid % HD (the strides NT / F4 and 4 * NT / HD are whole pages of keys).
+    // column kcol, its V slots rows 4 * (tid / HDL) % 16 .. +3 at column
+    // vcol (the strides NT / F4 and 4 * NT / HDL are whole pages of keys).
     // Each address is then one 32 x 32 -> 64-bit multiply-add on a base fixed
     // for the launch, where the page stride in bytes fits 32 bits (a page of
     // 16 rows over every layer is far below 4 GiB in practice; otherwise
     // fetch_with runs).
-    static_assert((NT / F4) % 16 == 0 && (4 * NT / HD) % 16 == 0 && BNM % 16 == 0,
+    // (A 256-wide row leaves 8 rows per stride: odd loads are then 8 rows on.)
+    constexpr int KSTEP = (NT / F4) % 16, VSTEP = (4 * NT / HDL) % 16;
+    static_assert(BNM % 16 == 0 && ((KSTEP == 0 && VSTEP == 0) || (APPEND == 0 && NT / F4 == 8 && 4 * NT / HDL == 8)),
                   "a thread's rows within a page are the same in every tile");
     const uint32_t stride_b = (uint32_t)((uint64_t)a.page_stride * sizeof(float));
     const char* const kb = reinterpret_cast<const char*>(
-        kbase + (size_t)((threadIdx.x / F4) % 16) * a.kv_dim + (threadIdx.x % F4) * 4);
+        kbase + (size_t)((threadIdx.x / F4) % 16) * a.kv_dim + kcol);
     const char* const vb = reinterpret_cast<const char*>(
-        vbase + (size_t)((4 * (threadIdx.x / HD)) % 16) * a.kv_dim + threadIdx.x % HD);
+        vbase + (size_t)((4 * (threadIdx.x / HDL)) % 16) * a.kv_dim + vcol);
     const size_t vrow_b = (size_t)a.kv_dim * sizeof(float);
-    // FULL: every key of the tile is at most last_pos (wave-uniform), so
+    // WHOLE: every key of the tile is at most last_pos (wave-uniform), so
     // only the page ids decide validity and no index needs clamping.
     // SRC: the keys are read from the pool (POOL) or, in an APPEND launch,
     // from the new rows (NEW), where the sequence's row j holds position
@@ -777,13 +808,13 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
     // so the address is one per-thread base (kn, vn) plus a block-uniform
     // multiple of the 16-row pitch (scalar arithmetic).
     const char* const kn = kb + dk + (size_t)(uint32_t)((threadIdx.x / F4) >> 4) * rows16_b;
-    const char* const vn = vb + dv + (size_t)(uint32_t)((4 * (threadIdx.x / HD)) >> 4) * rows16_b;
+    const char* const vn = vb + dv + (size_t)(uint32_t)((4 * (threadIdx.x / HDL)) >> 4) * rows16_b;
     auto fetch_lds_as = [&](int tile, auto full, auto src) __attribute__((always_inline)) {
-        constexpr bool FULL = decltype(full)::value;
+        constexpr bool WHOLE = decltype(full)::value;
         constexpr int SRC = decltype(src)::value;
-        if constexpr (SRC == NEW && FULL) {
-            kmask = KFULL;
-            vmask = VFULL;
+        if constexpr (SRC == NEW && WHOLE) {
+            kmask = kreal ? KFULL : 0;
+            vmask = vreal ? VFULL : 0;
             // (readfirstlane keeps each page index opaque: folded into kn / vn,
             // the compiler holds a 64-bit base per load and spills them)
 #pragma unroll
@@ -793,7 +824,7 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
             }
 #pragma unroll
             for (int i = 0; i < VSLOTS; i++) {
-                const int pg = __builtin_amdgcn_readfirstlane(tile * (BNM / 16) + i * (4 * NT / HD / 16));
+                const int pg = __builtin_amdgcn_readfirstlane(tile * (BNM / 16) + i * (4 * NT / HDL / 16));
                 const char* p = vn + (size_t)(uint32_t)pg * rows16_b;
 #pragma unroll
                 for (int e = 0; e < 4; e++) vreg[i][e] = *reinterpret_cast<const float*>(p + e * vrow_b);
@@ -804,11 +835,11 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
 #pragma unroll
         for (int i = 0; i < LOADS; i++) {
             const int key = tile * BNM + (int)(threadIdx.x + i * NT) / F4;
-            const int kc = FULL ? key : min(key, last_pos);
+            const int kc = WHOLE ? key : min(key, last_pos);
             const int page = SRC == NEW ? 0 : s_table[kc >> 4];  // -1: outside the pool
-            const bool ok = (FULL || key <= last_pos) && page >= 0;
-            kmask |= (uint32_t)ok << i;
-            const size_t pool_off = (size_t)(uint32_t)(ok ? page : 0) * stride_b;
+            const bool ok = (WHOLE || key <= last_pos) && page >= 0;
+            kmask |= (uint32_t)(ok && kreal) << i;
+            const size_t pool_off = (size_t)(uint32_t)(ok ? page : 0) * stride_b + (i * KSTEP % 16) * vrow_b;
             const size_t new_off = dk + (size_t)(uint32_t)(kc >> 4) * rows16_b;
             const size_t off = SRC == POOL                  ? pool_off
                                : SRC == MIXED && kc < start ? pool_off
@@ -817,24 +848,24 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
         }
 #pragma unroll
         for (int i = 0; i < VSLOTS; i++) {
-            const int key0 = tile * BNM + 4 * ((int)(threadIdx.x + i * NT) / HD);  // 4 keys, one page
-            const int kc = FULL ? key0 : min(key0, last_pos);
+            const int key0 = tile * BNM + 4 * ((int)(threadIdx.x + i * NT) / HDL);  // 4 keys, one page
+            const int kc = WHOLE ? key0 : min(key0, last_pos);
             const int page = SRC == NEW ? 0 : s_table[kc >> 4];
-            const bool ok = (FULL || key0 <= last_pos) && page >= 0;
-            const char* vp = vb + (size_t)(uint32_t)(ok ? page : 0) * stride_b;
+            const bool ok = (WHOLE || key0 <= last_pos) && page >= 0;
+            const char* vp = vb + (size_t)(uint32_t)(ok ? page : 0) * stride_b + (i * VSTEP % 16) * vrow_b;
             const char* vn = vb + (ok ? dv + (size_t)(uint32_t)(kc >> 4) * rows16_b : 0);
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 // a new row past last_pos is not read (the sequence's rows end there)
-                const int ec = FULL ? e : max(0, min(e, last_pos - key0));
+                const int ec = WHOLE ? e : max(0, min(e, last_pos - key0));
                 const char* p = SRC == POOL || (SRC == MIXED && key0 + e < start) ? vp + e * vrow_b : vn + ec * vrow_b;
                 vreg[i][e] = *reinterpret_cast<const float*>(p);
             }
-            if (FULL) {
-                vmask |= (ok ? 0xFu : 0u) << (4 * i);
+            if (WHOLE) {
+                vmask |= (ok && vreal ? 0xFu : 0u) << (4 * i);
             } else {
 #pragma unroll
-                for (int e = 0; e < 4; e++) vmask |= (uint32_t)(ok && key0 + e <= last_pos) << (4 * i + e);
+                for (int e = 0; e < 4; e++) vmask |= (uint32_t)(ok && vreal && key0 + e <= last_pos) << (4 * i + e);
             }
         }
     };
@@ -934,7 +965,7 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
                 const bool ok = !masked || ((kmask >> i) & 1);
                 const float kv4[4] = {ok ? kreg[i].x : 0.f, ok ? kreg[i].y : 0.f, ok ? kreg[i].z : 0.f,
                                       ok ? kreg[i].w : 0.f};
-                stage4(&k_lds[r * KST + col * 4], KPLANE, kv4);
+                if (HDL == HD || col * 4 < HD) stage4(&k_lds[r * KST + col * 4], KPLANE, kv4);
             }
 #pragma unroll
             for (int i = 0; i < VSLOTS; i++) {
@@ -942,7 +973,13 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
                 float v4[4];
 #pragma unroll
                 for (int e = 0; e < 4; e++) v4[e] = !masked || ((vmask >> (4 * i + e)) & 1) ? vreg[i][e] : 0.f;
-                stage4v(&v_lds[(sl % HD) * VST + 4 * (sl / HD)], VPLANE, v4);
+                if (HDL == HD || vslot < HD) {
+                    uint16_t* dst = &v_lds[vslot * VST + 4 * (sl / HDL)];
+                    if constexpr (VP == 3)
+                        stage4(dst, VPLANE, v4);
+                    else
+                        stage4v(dst, VPLANE, v4);
+                }
             }
         };
         if constexpr (APPEND == 1) {
@@ -954,7 +991,7 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
                 }
 #pragma unroll
                 for (int i = 0; i < VSLOTS; i++) {
-                    const int key0 = tile * BNM + 4 * ((int)(threadIdx.x + i * NT) / HD);  // 4 keys, one page
+                    const int key0 = tile * BNM + 4 * ((int)(threadIdx.x + i * NT) / HDL);  // 4 keys, one page
                     if (s_table[min(key0, last_pos) >> 4] < 0) vmask &= ~(0xFu << (4 * i));
                 }
             }
@@ -979,22 +1016,22 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
                 for (int i = 0; i < LOADS; i++) {
                     const int f = threadIdx.x + i * NT;
                     const int key = tile * BNM + f / F4;
-                    if (key >= own_first && key <= last_pos) {
+                    if (kcol_ok && key >= own_first && key <= last_pos) {
                         const int page = s_table[key >> 4];
                         if (page >= 0)
                             __builtin_nontemporal_store(f32x4{kreg[i].x, kreg[i].y, kreg[i].z, kreg[i].w},
                                                         reinterpret_cast<f32x4*>(kw + (size_t)(uint32_t)page * stride_b));
-                        else if (kv_h == 0 && f % F4 == 0)
+                        else if (kv_h == 0 && kslot == 0)
                             atomicAdd(a.bad_pages, 1);
                     }
                 }
 #pragma unroll
                 for (int i = 0; i < VSLOTS; i++) {
-                    const int key0 = tile * BNM + 4 * ((int)(threadIdx.x + i * NT) / HD);  // 4 keys, one page
+                    const int key0 = tile * BNM + 4 * ((int)(threadIdx.x + i * NT) / HDL);  // 4 keys, one page
                     const int page = s_table[min(key0, last_pos) >> 4];
 #pragma unroll
                     for (int e = 0; e < 4; e++)
-                        if (key0 + e >= own_first && key0 + e <= last_pos && page >= 0)
+                        if (vcol_ok && key0 + e >= own_first && key0 + e <= last_pos && page >= 0)
                             __builtin_nontemporal_store(
                                 vreg[i][e], reinterpret_cast<float*>(vw + (size_t)(uint32_t)page * stride_b + e * vrow_b));
                 }
@@ -1015,18 +1052,21 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
                 st[j] = f32x4{0.f, 0.f, 0.f, 0.f};
                 if (j < nvb) {  // wave-uniform
                     const uint16_t* kr = &k_lds[((kg + j * KSPLIT) * 16 + ql) * KST + 8 * g];
+                    f32x4 small = st[j];  // VP 3: the five small products apart, added once
 #pragma unroll
                     for (int c = 0; c < NC; c++) {
                         const bf16x8 kh = *reinterpret_cast<const bf16x8*>(kr + 32 * c);
                         const bf16x8 km = *reinterpret_cast<const bf16x8*>(kr + KPLANE + 32 * c);
                         const bf16x8 kl = *reinterpret_cast<const bf16x8*>(kr + 2 * KPLANE + 32 * c);
-                        st[j] = mfma(kl, qp[0][c], st[j]);
-                        st[j] = mfma(km, qp[1][c], st[j]);
-                        st[j] = mfma(kh, qp[2][c], st[j]);
-                        st[j] = mfma(km, qp[0][c], st[j]);
-                        st[j] = mfma(kh, qp[1][c], st[j]);
+                        f32x4& t = VP == 3 ? small : st[j];
+                        t = mfma(kl, qp[0][c], t);
+                        t = mfma(km, qp[1][c], t);
+                        t = mfma(kh, qp[2][c], t);
+                        t = mfma(km, qp[0][c], t);
+                        t = mfma(kh, qp[1][c], t);
                         st[j] = mfma(kh, qp[0][c], st[j]);
                     }
+                    if constexpr (VP == 3) st[j] += small;
                 }
             }
             const int last_key0 = tile * BNM + (kg + (nvb - 1) * KSPLIT) * 16;
@@ -1083,16 +1123,19 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
                 if (2 * jj < nvb) {  // wave-uniform
                     const float pv[8] = {p[2 * jj][0],     p[2 * jj][1],     p[2 * jj][2],     p[2 * jj][3],
                                          p[2 * jj + 1][0], p[2 * jj + 1][1], p[2 * jj + 1][2], p[2 * jj + 1][3]};
-                    bf16x8 ph, pm;
-                    split2(pv, ph, pm);
+                    bf16x8 ph, pm, pl;
+                    if constexpr (VP == 3)
+                        split3(pv, ph, pm, pl);
+                    else
+                        split2(pv, ph, pm);
                     const int key_a = (kg + 2 * jj * KSPLIT) * 16 + 4 * g;        // within the tile
                     const int key_b = (kg + (2 * jj + 1) * KSPLIT) * 16 + 4 * g;
 #pragma unroll
                     for (int n = 0; n < NB; n++) {
                         const uint16_t* vr = &v_lds[(16 * n + ql) * VST];
-                        bf16x8 vp[2];
+                        bf16x8 vp[VP];
 #pragma unroll
-                        for (int q = 0; q < 2; q++) {
+                        for (int q = 0; q < VP; q++) {
                             const uint2 x0 = *reinterpret_cast<const uint2*>(vr + q * VPLANE + key_a);
                             const uint2 x1 = *reinterpret_cast<const uint2*>(vr + q * VPLANE + key_b);
                             u32x4 t;
@@ -1100,7 +1143,13 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
                             vp[q] = __builtin_bit_cast(bf16x8, t);
                         }
                         f32x4 o = acc[n];
-                        o = mfma(vp[1], pm, o);
+                        if constexpr (VP == 3) {
+                            o = mfma(vp[2], ph, o);
+                            o = mfma(vp[1], pm, o);
+                            o = mfma(vp[0], pl, o);
+                        } else {
+                            o = mfma(vp[1], pm, o);
+                        }
                         o = mfma(vp[1], ph, o);
                         o = mfma(vp[0], pm, o);
                         o = mfma(vp[0], ph, o);
@@ -1148,29 +1197,47 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
     }
     if (row < qcount) {
         const float inv = 1.0f / lsum;
-        float* op = a.out + qrow * dim + (size_t)h * HD;
+        float* op = a.out + qrow * dim + (size_t)h * hd;
 #pragma unroll
         for (int n = 0; n < NB; n++)
-            *reinterpret_cast<float4*>(op + 16 * n + 4 * g) =
-                make_float4(acc[n][0] * inv, acc[n][1] * inv, acc[n][2] * inv, acc[n][3] * inv);
+            if (FULL || 16 * n + 4 * g < hd)
+                *reinterpret_cast<float4*>(op + 16 * n + 4 * g) =
+                    make_float4(acc[n][0] * inv, acc[n][1] * inv, acc[n][2] * inv, acc[n][3] * inv);
     }
+}
+
+// One instance of the bf16 matrix-core kernel; APPENDS: its appending forms are built.
+template <int HDL, int HD, bool FULL, int VP, int QT, int KSPLIT, int BNM, bool APPENDS>
+void launch_x3(const PrefillLaunch& a, dim3 grid, hipStream_t stream) {
+    const dim3 block(64 * QT * KSPLIT);
+    if constexpr (APPENDS) {
+        if (a.k_new && a.append_mixed)
+            hipLaunchKernelGGL((paged_attn_prefill_x3_kernel<HDL, HD, FULL, VP, QT, KSPLIT, BNM, 2>), grid, block, 0, stream, a);
+        else if (a.k_new)
+            hipLaunchKernelGGL((paged_attn_prefill_x3_kernel<HDL, HD, FULL, VP, QT, KSPLIT, BNM, 1>), grid, block, 0, stream, a);
+        if (a.k_new) return;
+    }
+    hipLaunchKernelGGL((paged_attn_prefill_x3_kernel<HDL, HD, FULL, VP, QT, KSPLIT, BNM, 0>), grid, block, 0, stream, a);
 }
 
 }  // namespace
 
 int prefill_block_m(int) { return BM; }
 
-// hd 128 runs one key group per workgroup (its registers), so 128-row items
-// (8 waves, each staged tile serving 128 queries) measured 15-20% faster
-// than 64-row ones.  At hd 64 the 64-row items of two key groups are kept:
+// Heads past 64 run one key group per workgroup (its registers), so 128-row
+// items (8 waves, each staged tile serving 128 queries) measured 15-20% faster
+// than 64-row ones at hd 128, and at hd 96 with 4-wave workgroups, three to a
+// CU, 6% (one 4000-token prompt; 2% on 6 prompts of 50-700 tokens, 2-4% slower
+// on two 100-300 token chunks after cached keys).  At hd 64 the 64-row items of two key groups are kept:
 // 128-row items there need 16-wave workgroups, one per CU, and measured 9%
 // slower on the 8-prompt mix (faster on large balanced batches).
 bool prefill_uses_wide_items(int32_t kernel, int32_t head_dim) {
-    return kernel == PREFILL_KERNEL_DEFAULT && head_dim == 128;
+    return kernel == PREFILL_KERNEL_DEFAULT && head_dim > 64;
 }
 
 bool prefill_appends_in_launch(int32_t kernel, int32_t head_dim, int32_t max_pos, int64_t page_stride) {
-    return kernel == PREFILL_KERNEL_DEFAULT && (head_dim == 32 || head_dim == 64 || head_dim == 128) &&
+    const bool built = head_dim == 32 || head_dim == 64 || head_dim == 128 || (head_dim > 64 && head_dim <= 96);
+    return kernel == PREFILL_KERNEL_DEFAULT && built &&
            (max_pos >> 4) < TABLE_LDS && (uint64_t)page_stride * sizeof(float) < (1ull << 32);
 }
 
@@ -1182,29 +1249,23 @@ hipError_t launch_paged_attn_prefill(const PrefillLaunch& a, hipStream_t stream)
     if ((a.k_new != nullptr) != (a.v_new != nullptr) ||
         (a.k_new && !prefill_appends_in_launch(a.kernel, a.head_dim, a.max_pos, a.page_stride)))
         return hipErrorInvalidValue;  // only the bf16 matrix-core kernel appends, with the table in LDS
-    if (a.kernel == PREFILL_KERNEL_DEFAULT && a.k_new && !a.append_mixed) {
-        switch (a.head_dim) {
-            case 32: hipLaunchKernelGGL((paged_attn_prefill_x3_kernel<32, 4, 2, 64, 1>), grid, dim3(512), 0, stream, a); return hipGetLastError();
-            case 64: hipLaunchKernelGGL((paged_attn_prefill_x3_kernel<64, 4, 2, 64, 1>), grid, dim3(512), 0, stream, a); return hipGetLastError();
-            case 128: hipLaunchKernelGGL((paged_attn_prefill_x3_kernel<128, 8, 1, 32, 1>), grid, dim3(512), 0, stream, a); return hipGetLastError();
-            default: return hipErrorInvalidValue;
-        }
-    }
-    if (a.kernel == PREFILL_KERNEL_DEFAULT && a.k_new) {
-        switch (a.head_dim) {
-            case 32: hipLaunchKernelGGL((paged_attn_prefill_x3_kernel<32, 4, 2, 64, 2>), grid, dim3(512), 0, stream, a); return hipGetLastError();
-            case 64: hipLaunchKernelGGL((paged_attn_prefill_x3_kernel<64, 4, 2, 64, 2>), grid, dim3(512), 0, stream, a); return hipGetLastError();
-            case 128: hipLaunchKernelGGL((paged_attn_prefill_x3_kernel<128, 8, 1, 32, 2>), grid, dim3(512), 0, stream, a); return hipGetLastError();
-            default: return hipErrorInvalidValue;
-        }
-    }
     if (a.kernel == PREFILL_KERNEL_DEFAULT) {
-        switch (a.head_dim) {
-            case 32: hipLaunchKernelGGL((paged_attn_prefill_x3_kernel<32, 4, 2, 64, 0>), grid, dim3(512), 0, stream, a); return hipGetLastError();
-            case 64: hipLaunchKernelGGL((paged_attn_prefill_x3_kernel<64, 4, 2, 64, 0>), grid, dim3(512), 0, stream, a); return hipGetLastError();
-            case 128: hipLaunchKernelGGL((paged_attn_prefill_x3_kernel<128, 8, 1, 32, 0>), grid, dim3(512), 0, stream, a); return hipGetLastError();
-            default: break;  // other head sizes: VALU kernel
-        }
+        // The appending forms are built where a batch's fresh prompts are the
+        // usual call at that size: 32, 64, 96 and 128 wide (the scatter in
+        // front took 15 of 85 us per layer at 16 x 96).
+        const int hd = a.head_dim;
+        if (hd < 4 || hd > 256 || hd % 4) return hipErrorInvalidValue;
+        if (hd == 32) launch_x3<32, 32, true, 2, 4, 2, 64, true>(a, grid, stream);
+        else if (hd == 64) launch_x3<64, 64, true, 2, 4, 2, 64, true>(a, grid, stream);
+        else if (hd == 128) launch_x3<128, 128, true, 2, 8, 1, 32, true>(a, grid, stream);
+        else if (hd == 96) launch_x3<128, 96, true, 3, 8, 1, 32, true>(a, grid, stream);
+        else if (hd == 256) launch_x3<256, 256, true, 3, 8, 1, 32, false>(a, grid, stream);
+        else if (hd < 32) launch_x3<32, 32, false, 3, 4, 2, 64, false>(a, grid, stream);
+        else if (hd < 64) launch_x3<64, 64, false, 3, 4, 2, 64, false>(a, grid, stream);
+        else if (hd < 96) launch_x3<128, 96, false, 3, 8, 1, 32, true>(a, grid, stream);
+        else if (hd < 128) launch_x3<128, 128, false, 3, 8, 1, 32, false>(a, grid, stream);
+        else launch_x3<256, 256, false, 3, 8, 1, 32, false>(a, grid, stream);
+        return hipGetLastError();
     }
     if (a.kernel == PREFILL_KERNEL_MFMA_F32) {
         // 4 query sub-tiles x 2 key groups per workgroup, one workgroup per
@@ -1218,8 +1279,7 @@ hipError_t launch_paged_attn_prefill(const PrefillLaunch& a, hipStream_t stream)
             default: break;  // other head sizes: VALU kernel
         }
     }
-    // VALU kernel: hd 256, head sizes other than 32/64/128/256 (padded), or
-    // NITRO_PREFILL_KERNEL=valu
+    // VALU kernel: NITRO_PREFILL_KERNEL=valu, and mfma32 at other head sizes
     if (a.head_dim < 4 || a.head_dim > 256 || a.head_dim % 4) return hipErrorInvalidValue;
     const int hdp = a.head_dim <= 32 ? 32 : a.head_dim <= 64 ? 64 : a.head_dim <= 128 ? 128 : 256;
     const bool full = a.head_dim == hdp;

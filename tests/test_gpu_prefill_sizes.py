@@ -1,0 +1,71 @@
+"""Prefill attention at head sizes around the widths its kernels are built for
+(32, 64, 96, 128, 256 columns): fresh prompts, chunks after cached keys, ragged
+lengths around the query and key tiles, grouped-query heads, against 64-bit
+attention.  The scatter + attention pair and the append call agree exactly."""
+import numpy as np
+import pytest
+
+from gpu_helpers import to_gpu
+from test_gpu_prefill import prefill_batch_case
+
+pytestmark = pytest.mark.gpu
+
+
+def exact(c, k, v):
+    """Causal attention in 64 bits over the appended pools."""
+    H, Hkv, hd, layer = c["H"], c["Hkv"], c["hd"], c["layer"]
+    out, row = np.zeros(c["q"].shape), 0
+    for b, (start, n) in enumerate(zip(c["starts"], c["lens"])):
+        pos = np.arange(int(start + n))
+        kk, vv = (p[c["tables"][b][pos // 16], layer, pos % 16].astype(np.float64).reshape(len(pos), Hkv, hd) for p in (k, v))
+        q = c["q"][row:row + n].astype(np.float64).reshape(int(n), H, hd)
+        seen = pos[None, :] <= int(start) + np.arange(int(n))[:, None]
+        for h in range(H):
+            s = np.where(seen, q[:, h] @ kk[:, h * Hkv // H].T / np.sqrt(hd), -np.inf)
+            p = np.exp(s - s.max(axis=1, keepdims=True))
+            out[row:row + n, h * hd:(h + 1) * hd] = (p / p.sum(axis=1, keepdims=True)) @ vv[:, h * Hkv // H]
+        row += int(n)
+    return out
+
+
+def run(c, append):
+    import torch
+
+    import nitrorag_amd as na
+
+    k, v = to_gpu(c["k"]), to_gpu(c["v"])
+    pool = na.KVPool.wrap(k, v)
+    pool.upload_prefill_batch(c["tables"], c["starts"], c["lens"])
+    q, kc, vc = to_gpu(c["q"]), to_gpu(c["kc"]), to_gpu(c["vc"])
+    out = torch.full_like(q, float("nan"))
+    if append:
+        pool.prefill_append(c["layer"], q, kc, vc, out, c["H"], c["Hkv"], c["hd"])
+    else:
+        pool.kv_append_prefill(c["layer"], kc, vc)
+        pool.prefill(c["layer"], q, out, c["H"], c["Hkv"], c["hd"])
+    torch.cuda.synchronize()
+    assert pool.take_device_errors() == 0
+    return out.cpu().numpy(), k.cpu().numpy(), v.cpu().numpy()
+
+
+# (lengths lo, hi, starts lo, hi): single tokens, around a key tile (32, 64) and
+# a query item (64, 128), chunks after cached keys that start inside a page
+SHAPES = [(1, 1, 0, 0), (31, 33, 0, 0), (127, 130, 0, 0), (1, 140, 1, 200)]
+
+
+@pytest.mark.parametrize("hd", [4, 28, 36, 60, 68, 80, 92, 96, 100, 124, 132, 252, 256])
+def test_head_sizes(hd):
+    for i, (lo, hi, slo, shi) in enumerate(SHAPES):
+        print(f"prefill hd {hd} lengths {lo}-{hi} after {slo}-{shi}", flush=True)
+        c = prefill_batch_case(100 + i, 3, lo, hi, 4, 2, hd, 2, 1, slo, shi)
+        got, gk, gv = run(c, False)
+        fused, fk, fv = run(c, True)
+        assert np.array_equal(got, fused) and np.array_equal(gk, fk) and np.array_equal(gv, fv)
+        want = exact(c, gk, gv)
+        # fp32 sums: a score (below 8 in size here, its error enters the weights
+        # directly) is a sum of hd products and an output one of at most 340
+        # weighted values; each term is rounded to 2^-24 and independent roundings
+        # add as their root, twice which bounds the 2-norm
+        bound = 2 * np.sqrt(8 * hd + 340) * 2.0 ** -24
+        err = np.linalg.norm(got - want) / np.linalg.norm(want)
+        assert err <= bound, (hd, lo, hi, err, bound)
