@@ -24,7 +24,7 @@ LIB = os.path.join(HERE, "libnitro_paged_attn.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("NITRO_OFFLOAD_ARCH", "gfx950")
-DEVICE_SOURCES = ["paged_attn_decode.hip", "paged_attn_prefill.hip", "kv_append.hip", "q8_matmul.hip",
+DEVICE_SOURCES = ["paged_attn_decode.hip", "paged_attn_prefill.hip", "kv_append.hip", "q8_matmul.hip", "q8_gemm.hip",
                   "model_kernels.hip", "scheduler_kernels.hip"]
 HIP_HOST_SOURCES = ["capi_device.cpp", "model.cpp", "scheduler_step.cpp"]
 HOST_SOURCES = ["paged_memory.cpp", "capi_host.cpp", "scheduler.cpp", "rpc.cpp"]

@@ -302,6 +302,11 @@ struct Q8Tiled {
 // rows; products of more full rows read the tile layout when there is one.
 constexpr int Q8_GEMV_MAX_BATCH = 4;
 inline size_t q8_tiled_bytes(size_t d, size_t n) { return (d + 15) / 16 * (n / 32) * 576; }
+// Activations of a large product in split form: per 16 rows and 32-k block
+// three planes (hi, mid, lo bf16 parts) of 64 runs of 8 k, run l holding row
+// l%16, k = 8*(l/16) .. +8: the operand order of v_mfma_f32_16x16x32_bf16.
+constexpr int Q8_SPLIT_BYTES = 3072;
+inline size_t q8_split_bytes(size_t rows, size_t n) { return (rows + 15) / 16 * (n / 32) * Q8_SPLIT_BYTES; }
 // tiled = the tile layout of w (rows of BlockQ8, d x n)
 hipError_t launch_q8_tile(const void* w, void* tiled, int d, int n, hipStream_t stream);
 // Q8_0 matrix product (rows of BlockQ8, fp32 activations); last_block_only
@@ -311,17 +316,17 @@ hipError_t launch_q8_matmul(const void* w, const float* x, float* out, int batch
 // x[b] += w . in[b] ([batch][d], in place) with the squares of the new x
 // rows summed per 16 outputs into ss (ceil(d/16) partials per row, stride batch).
 hipError_t launch_q8_residual(const void* w, const float* in, float* x, float* ss, int batch, int n, int d,
-                              bool last_block_only, hipStream_t stream, const void* w_tiled = nullptr);
+                              bool last_block_only, hipStream_t stream, const void* w_tiled = nullptr, void* split = nullptr);
 // wq/wk/wv sharing x and n: q = wq . rms_norm(x), k, v likewise, with the
 // RoPE + K/V-append epilogue: q written to out_q [batch][dim], k and v to the
 // pools (d = {dim, kv_dim, kv_dim}).
 hipError_t launch_q8_qkv(const void* const* w, const float* x, float* out_q, const int* d, int batch, int n,
                          bool last_block_only, const Q8Norm& norm, const Q8Rope& rope, hipStream_t stream,
-                         const Q8Tiled& tiled = Q8Tiled{});
+                         const Q8Tiled& tiled = Q8Tiled{}, void* split = nullptr);
 // hb = silu(x . w1^T) * (x . w3^T), [batch][hidden] (src/model_q8.cpp:670-680).
 hipError_t launch_q8_swiglu(const void* w1, const void* w3, const float* x, float* hb, int batch, int n,
                             int hidden, bool last_block_only, const Q8Norm& norm, hipStream_t stream,
-                            const Q8Tiled& tiled = Q8Tiled{});
+                            const Q8Tiled& tiled = Q8Tiled{}, void* split = nullptr);
 // Row-wise model kernels and the fp32 classifier product (model_kernels.hip).
 // x[r] = table[tokens[r]]; with ss, ss[r] = the row's sum of squares (one
 // partial per row for a following Q8Norm).

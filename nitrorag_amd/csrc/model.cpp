@@ -32,6 +32,7 @@ struct nitro_model {
     size_t tiled_bytes = 0;
     size_t t_wq = 0, t_wk = 0, t_wv = 0, t_wo = 0, t_w1 = 0, t_w2 = 0, t_w3 = 0;
     DeviceBuffer<float> x, attn, q, hb, last, ss;
+    DeviceBuffer<uint8_t> split;  // a product's activations in split form (many rows)
     DeviceBuffer<int32_t> tokens;
     Staging staging;
 
@@ -87,6 +88,7 @@ void reserve_rows(nitro_model* m, int rows) {
     m->q.reserve(r * m->dim);
     m->hb.reserve(r * m->hidden);
     m->tokens.reserve(r);
+    if (rows > 64) m->split.reserve(q8_split_bytes(r, (size_t)std::max(m->dim, m->hidden)));
 }
 
 void check_model_pool(const nitro_model* m, const nitro_kvpool* pool) {
@@ -139,6 +141,7 @@ void layers(nitro_model* m, nitro_kvpool* pool, const int32_t* tokens, int rows,
     hip_check(launch_embed_rows(m->f32(m->o_emb), tokens, m->x.ptr, rows, dim, m->vocab, pool->bad_pages.ptr,
                                 m->ss.ptr, s),
               "embed launch");
+    void* const split = rows > 64 ? m->split.ptr : nullptr;
     for (int l = 0; l < m->n_layers; l++) {
         // q, k, v = wq/wk/wv . rms_norm(x, rms_att) in one launch, RoPE on q and
         // k, k and v appended to the pools (:586-617)
@@ -151,12 +154,12 @@ void layers(nitro_model* m, nitro_kvpool* pool, const int32_t* tokens, int rows,
         tqkv.w[2] = m->q8t(m->t_wv, l, kv, dim);
         const int dqkv[3] = {dim, kv, kv};
         rope.layer_off = pool->layer_offset(l);
-        hip_check(launch_q8_qkv(wqkv, m->x.ptr, m->q.ptr, dqkv, rows, dim, last, att, rope, s, tqkv),
+        hip_check(launch_q8_qkv(wqkv, m->x.ptr, m->q.ptr, dqkv, rows, dim, last, att, rope, s, tqkv, split),
                   "q8_qkv launch");
         attend(l);  // attention over the pools -> m->attn (:618-662)
         // x += wo . attn (:663-666)
         hip_check(launch_q8_residual(m->q8(m->o_wo, l, dim, dim), m->attn.ptr, m->x.ptr, m->ss.ptr, rows, dim,
-                                     dim, last, s, m->q8t(m->t_wo, l, dim, dim)),
+                                     dim, last, s, m->q8t(m->t_wo, l, dim, dim), split),
                   "q8 wo launch");
         // hb = silu(w1 . xb) * (w3 . xb), xb = rms_norm(x, rms_ffn), one launch (:667-680)
         const Q8Norm ffn{m->f32(m->o_rms_ffn) + (size_t)l * dim, m->ss.ptr, parts, rows};
@@ -164,11 +167,11 @@ void layers(nitro_model* m, nitro_kvpool* pool, const int32_t* tokens, int rows,
         t13.w[0] = m->q8t(m->t_w1, l, hid, dim);
         t13.w[1] = m->q8t(m->t_w3, l, hid, dim);
         hip_check(launch_q8_swiglu(m->q8(m->o_w1, l, hid, dim), m->q8(m->o_w3, l, hid, dim), m->x.ptr,
-                                   m->hb.ptr, rows, dim, hid, last, ffn, s, t13),
+                                   m->hb.ptr, rows, dim, hid, last, ffn, s, t13, split),
                   "q8_swiglu launch");
         // x += w2 . hb (:682-684)
         hip_check(launch_q8_residual(m->q8(m->o_w2, l, dim, hid), m->hb.ptr, m->x.ptr, m->ss.ptr, rows, hid,
-                                     dim, last, s, m->q8t(m->t_w2, l, dim, hid)),
+                                     dim, last, s, m->q8t(m->t_w2, l, dim, hid), split),
                   "q8 w2 launch");
     }
 }

@@ -18,7 +18,9 @@
 //  - full rows, 1..4 rows: VALU dot products.  Rows of >= 2048 k take
 //    q8_flat_kernel when the activations fit its LDS (batch x n <= 16384
 //    floats), else q8_rowdot_kernel; q8_gemv_kernel covers short rows.
-//  - full rows, more rows: q8_mma_kernel, the bf16 matrix cores at fp32
+//  - full rows, many rows: q8_gemm_kernel (q8_gemm.hip), where a launch has
+//    the outputs to fill it.
+//  - full rows, more than 4 rows otherwise: q8_mma_kernel, the bf16 matrix cores at fp32
 //    accuracy (x split into three exact bf16 parts), over the model's
 //    tile-layout copy of the matrix when there is one (Q8Tiled) or the BlockQ8
 //    rows otherwise; q8_matmul_kernel on v_mfma_f32_16x16x4_f32 under
@@ -48,14 +50,13 @@
 
 #include "bf16_split.hpp"
 #include "device_pool.hpp"
+#include "q8_group.hpp"
 
 namespace nitro {
 namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int Q8_BLOCK = 32;         // weights per block
-constexpr int Q8_BLOCK_BYTES = 36;   // float scale + 32 int8
 constexpr int Q8_WAVES = 4;
 constexpr int Q8_MAX_BTILES = 4;     // batch tiles of 16 per launch row (batch <= 64 per grid.y)
 constexpr int Q8_UNROLL = 4;         // 64-weight chunks whose loads a wave issues together
@@ -98,9 +99,6 @@ __device__ __forceinline__ float sum_over_rows(float x) {
     return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
-// Weight j (0..3) of a word of int8 weights, as a float.
-__device__ __forceinline__ float q8_value(uint32_t w, int j) { return (float)(int)(int8_t)(w >> (8 * j)); }
-
 __device__ __forceinline__ float dequant(uint32_t q4, int j, float scale) {
     return (float)(int)(int8_t)(q4 >> (8 * j)) * scale;
 }
@@ -122,64 +120,6 @@ __device__ __forceinline__ float partial_sum(const Q8Norm& nm, int b, int first,
     }
     return s;
 }
-
-// partial_sum with no branch around its loads: an index past the end rereads
-// the last partial and adds 0 (same order of adds), so all L loads of a round
-// go out together, behind any loads issued before.
-template <int L>
-__device__ __forceinline__ float partial_sum_unbranched(const Q8Norm& nm, int b, int first, int step) {
-    float s = 0.0f;
-    for (int p0 = first; p0 < nm.nparts; p0 += L * step) {
-        float v[L];
-#pragma unroll
-        for (int i = 0; i < L; i++) v[i] = nm.ss[(size_t)min(p0 + i * step, nm.nparts - 1) * nm.ss_stride + b];
-#pragma unroll
-        for (int i = 0; i < L; i++) s += p0 + i * step < nm.nparts ? v[i] : 0.0f;
-    }
-    return s;
-}
-
-__device__ __forceinline__ float inv_rms(float ss, int n) { return 1.0f / sqrtf(ss / (float)n + 1e-5f); }
-
-// Where batch row b's K/V goes and the position it rotates with.
-struct RopeRow {
-    int pos, page, in_page;
-    bool page_ok;
-};
-
-__device__ __forceinline__ RopeRow rope_row(const Q8Rope& rp, int b) {
-    const int w = b < rp.split ? 0 : 1;
-    const int i = w ? b - rp.split : b;
-    RopeRow r;
-    r.pos = rp.pos[w][i];
-    const int slot = rp.slot[w][i];
-    r.page = slot >> 4;
-    r.in_page = slot & 15;
-    r.page_ok = r.page >= 0 && r.page < rp.num_pages;
-    return r;
-}
-
-// (x, y) rotated by the angle of pair f of position pos: the reference's
-// (x*fcr - y*fci, x*fci + y*fcr) (src/model_q8.cpp:600-612).
-__device__ __forceinline__ float2 rotate_pair(const Q8Rope& rp, int pos, int feature, float x, float y) {
-    const int f = (feature % rp.head_dim) >> 1;
-    const float c = rp.freq_real[(size_t)pos * (rp.head_dim >> 1) + f];
-    const float sn = rp.freq_imag[(size_t)pos * (rp.head_dim >> 1) + f];
-    return make_float2(x * c - y * sn, x * sn + y * c);
-}
-
-}  // namespace
-
-// Up to 3 matrices sharing x (same n); out[m] is [batch][d[m]]; wt[m] the
-// same matrix in the tile layout (or null).
-struct Q8Group {
-    const uint8_t* w[3];
-    float* out[3];
-    int d[3];
-    const uint8_t* wt[3];
-};
-
-namespace {
 
 // The epilogue of one 16 x 16 output tile held as fp32 MFMA accumulators: lane
 // l holds out^T[row0 + 4*(l/16) + j][bb] (j = 0..3) of each group member, bb
@@ -1568,7 +1508,7 @@ __global__ __launch_bounds__(64) void q8_tile_kernel(const uint8_t* __restrict__
 
 template <int NMAT, bool SWIGLU, bool NORM, bool RESID, bool ROPE = false>
 void launch_group(const Q8Group& grp, const float* x, int batch, int n, int dmax, bool last, const Q8Norm& nm,
-                  const Q8Resid& rs, hipStream_t stream, const Q8Rope& rp = Q8Rope{}) {
+                  const Q8Resid& rs, hipStream_t stream, const Q8Rope& rp = Q8Rope{}, void* split = nullptr) {
     const dim3 grid((unsigned)((dmax + 15) / 16),
                     (unsigned)((batch + 16 * Q8_MAX_BTILES - 1) / (16 * Q8_MAX_BTILES)));
     const dim3 block(64 * Q8_WAVES);
@@ -1586,6 +1526,8 @@ void launch_group(const Q8Group& grp, const float* x, int batch, int n, int dmax
         }
         return;
     }
+    constexpr Q8Epilogue EPI = ROPE ? Q8Epilogue::Rope : RESID ? Q8Epilogue::Residual : SWIGLU ? Q8Epilogue::SwiGlu : Q8Epilogue::Store;
+    if (use_mma() && launch_q8_gemm(EPI, grp, x, split, batch, n, nm, rs, rp, stream)) return;
     // the bf16 kernel addresses weights and x with 32-bit offsets
     const bool mma_fits = q8_tiled_bytes(dmax, n) < (1ull << 32) && (size_t)batch * n < (1ull << 32) &&
                           (!NORM || n <= MMA_NORM_MAX_N);
@@ -1620,19 +1562,19 @@ hipError_t launch_q8_matmul(const void* w, const float* x, float* out, int batch
 }
 
 hipError_t launch_q8_residual(const void* w, const float* in, float* x, float* ss, int batch, int n, int d,
-                              bool last_block_only, hipStream_t stream, const void* w_tiled) {
+                              bool last_block_only, hipStream_t stream, const void* w_tiled, void* split) {
     Q8Group grp{{static_cast<const uint8_t*>(w), nullptr, nullptr},
                 {x, nullptr, nullptr},
                 {d, 0, 0},
                 {static_cast<const uint8_t*>(w_tiled), nullptr, nullptr}};
     launch_group<1, false, false, true>(grp, in, batch, n, d, last_block_only, Q8Norm{}, Q8Resid{ss, batch},
-                                        stream);
+                                        stream, Q8Rope{}, split);
     return hipGetLastError();
 }
 
 hipError_t launch_q8_qkv(const void* const* w, const float* x, float* out_q, const int* d, int batch, int n,
                          bool last_block_only, const Q8Norm& nm, const Q8Rope& rope, hipStream_t stream,
-                         const Q8Tiled& tiled) {
+                         const Q8Tiled& tiled, void* split) {
     if (!nm.weight || !rope.freq_real || d[1] != d[2] || d[0] % 32 || d[1] % 32) return hipErrorInvalidValue;
     Q8Group grp{};
     for (int m = 0; m < 3; m++) {
@@ -1642,19 +1584,19 @@ hipError_t launch_q8_qkv(const void* const* w, const float* x, float* out_q, con
     }
     grp.out[0] = out_q;  // k and v go to the pools
     const int dmax = std::max(d[0], d[1]);
-    launch_group<3, false, true, false, true>(grp, x, batch, n, dmax, last_block_only, nm, Q8Resid{}, stream, rope);
+    launch_group<3, false, true, false, true>(grp, x, batch, n, dmax, last_block_only, nm, Q8Resid{}, stream, rope, split);
     return hipGetLastError();
 }
 
 hipError_t launch_q8_swiglu(const void* w1, const void* w3, const float* x, float* hb, int batch, int n,
                             int hidden, bool last_block_only, const Q8Norm& nm, hipStream_t stream,
-                            const Q8Tiled& tiled) {
+                            const Q8Tiled& tiled, void* split) {
     Q8Group grp{{static_cast<const uint8_t*>(w1), static_cast<const uint8_t*>(w3), nullptr},
                 {hb, nullptr, nullptr},
                 {hidden, hidden, 0},
                 {static_cast<const uint8_t*>(tiled.w[0]), static_cast<const uint8_t*>(tiled.w[1]), nullptr}};
     if (!nm.weight) return hipErrorInvalidValue;
-    launch_group<2, true, true, false>(grp, x, batch, n, hidden, last_block_only, nm, Q8Resid{}, stream);
+    launch_group<2, true, true, false>(grp, x, batch, n, hidden, last_block_only, nm, Q8Resid{}, stream, Q8Rope{}, split);
     return hipGetLastError();
 }
 
