@@ -269,6 +269,13 @@ struct Q8Resid {
     float* ss = nullptr;
     int ss_stride = 0;
 };
+// A product's output left in split form for the next one (nb blocks a row),
+// each value times weight[its column] where weights are given.
+struct Q8SplitOut {
+    char* planes = nullptr;
+    const float* weight = nullptr;
+    int nb = 0;
+};
 // RoPE and the K/V append folded into the wq/wk/wv product's epilogue
 // (src/model_q8.cpp:594-617, 447-470): q and k are rotated with
 // freq_real/imag[pos] of their batch row, q goes to its buffer, k and v
@@ -302,11 +309,21 @@ struct Q8Tiled {
 // rows; products of more full rows read the tile layout when there is one.
 constexpr int Q8_GEMV_MAX_BATCH = 4;
 inline size_t q8_tiled_bytes(size_t d, size_t n) { return (d + 15) / 16 * (n / 32) * 576; }
-// Activations of a large product in split form: per 16 rows and 32-k block
-// three planes (hi, mid, lo bf16 parts) of 64 runs of 8 k, run l holding row
-// l%16, k = 8*(l/16) .. +8: the operand order of v_mfma_f32_16x16x32_bf16.
+// Activations in split form: per 16 rows and 32-k block three planes (hi, mid,
+// lo bf16 parts, an exact sum) of 64 runs of 8 k, run l holding row l%16, k =
+// 8*(l/16) .. +8: the operand order of v_mfma_f32_16x16x32_bf16.
 constexpr int Q8_SPLIT_BYTES = 3072;
 inline size_t q8_split_bytes(size_t rows, size_t n) { return (rows + 15) / 16 * (n / 32) * Q8_SPLIT_BYTES; }
+// Split activations of a product of more than 4 full rows in a model, whose
+// launches hand them on so that each value is split once, where it is made.
+struct Q8Split {
+    const void* in = nullptr;    // x, instead of the fp32 rows (with a Q8Norm: x times its weights; the sums take 1/rms)
+    Q8SplitOut out;              // left for the next product (the residual's x, SwiGLU's hb; hb then only here)
+    void* scratch = nullptr;     // without `in`: where a large product may split its fp32 x
+};
+// Whether the launches of a model with these widths may use split activations
+// at this many rows (32-bit offsets; the bf16 kernels selected).
+bool q8_split_usable(size_t rows, size_t dim, size_t hidden);
 // tiled = the tile layout of w (rows of BlockQ8, d x n)
 hipError_t launch_q8_tile(const void* w, void* tiled, int d, int n, hipStream_t stream);
 // Q8_0 matrix product (rows of BlockQ8, fp32 activations); last_block_only
@@ -316,22 +333,23 @@ hipError_t launch_q8_matmul(const void* w, const float* x, float* out, int batch
 // x[b] += w . in[b] ([batch][d], in place) with the squares of the new x
 // rows summed per 16 outputs into ss (ceil(d/16) partials per row, stride batch).
 hipError_t launch_q8_residual(const void* w, const float* in, float* x, float* ss, int batch, int n, int d,
-                              bool last_block_only, hipStream_t stream, const void* w_tiled = nullptr, void* split = nullptr);
+                              bool last_block_only, hipStream_t stream, const void* w_tiled = nullptr, const Q8Split& split = Q8Split{});
 // wq/wk/wv sharing x and n: q = wq . rms_norm(x), k, v likewise, with the
 // RoPE + K/V-append epilogue: q written to out_q [batch][dim], k and v to the
 // pools (d = {dim, kv_dim, kv_dim}).
 hipError_t launch_q8_qkv(const void* const* w, const float* x, float* out_q, const int* d, int batch, int n,
                          bool last_block_only, const Q8Norm& norm, const Q8Rope& rope, hipStream_t stream,
-                         const Q8Tiled& tiled = Q8Tiled{}, void* split = nullptr);
+                         const Q8Tiled& tiled = Q8Tiled{}, const Q8Split& split = Q8Split{});
 // hb = silu(x . w1^T) * (x . w3^T), [batch][hidden] (src/model_q8.cpp:670-680).
 hipError_t launch_q8_swiglu(const void* w1, const void* w3, const float* x, float* hb, int batch, int n,
                             int hidden, bool last_block_only, const Q8Norm& norm, hipStream_t stream,
-                            const Q8Tiled& tiled = Q8Tiled{}, void* split = nullptr);
+                            const Q8Tiled& tiled = Q8Tiled{}, const Q8Split& split = Q8Split{});
 // Row-wise model kernels and the fp32 classifier product (model_kernels.hip).
 // x[r] = table[tokens[r]]; with ss, ss[r] = the row's sum of squares (one
-// partial per row for a following Q8Norm).
+// partial per row for a following Q8Norm); with split.planes, x times
+// split.weight in split form.
 hipError_t launch_embed_rows(const float* table, const int32_t* tokens, float* x, int rows, int dim,
-                             int vocab, int32_t* bad_tokens, float* ss, hipStream_t stream);
+                             int vocab, int32_t* bad_tokens, float* ss, const Q8SplitOut& split, hipStream_t stream);
 hipError_t launch_add_rmsnorm(float* x, const float* delta, const float* weight, float* out, int rows,
                               int dim, hipStream_t stream);
 hipError_t launch_gather_last_rows(const float* x, const float* ffn, const int32_t* row_off,

@@ -32,7 +32,7 @@ struct nitro_model {
     size_t tiled_bytes = 0;
     size_t t_wq = 0, t_wk = 0, t_wv = 0, t_wo = 0, t_w1 = 0, t_w2 = 0, t_w3 = 0;
     DeviceBuffer<float> x, attn, q, hb, last, ss;
-    DeviceBuffer<uint8_t> split;  // a product's activations in split form (many rows)
+    DeviceBuffer<uint8_t> xsplit, hsplit;  // x (times the next norm's weights) and hb in split form
     DeviceBuffer<int32_t> tokens;
     Staging staging;
 
@@ -88,7 +88,10 @@ void reserve_rows(nitro_model* m, int rows) {
     m->q.reserve(r * m->dim);
     m->hb.reserve(r * m->hidden);
     m->tokens.reserve(r);
-    if (rows > 64) m->split.reserve(q8_split_bytes(r, (size_t)std::max(m->dim, m->hidden)));
+    if (q8_split_usable(r, m->dim, m->hidden)) {
+        m->xsplit.reserve(q8_split_bytes(r, m->dim));
+        m->hsplit.reserve(q8_split_bytes(r, (size_t)std::max(m->dim, m->hidden)));
+    }
 }
 
 void check_model_pool(const nitro_model* m, const nitro_kvpool* pool) {
@@ -138,10 +141,15 @@ void layers(nitro_model* m, nitro_kvpool* pool, const int32_t* tokens, int rows,
     const bool last = semantics == NITRO_Q8_LAST_BLOCK;
     const int parts = (dim + 15) / 16;  // partials per row left by wo / w2
     if (!last && rows > Q8_GEMV_MAX_BATCH) ensure_tiled(m, s);
+    // Products of more than 4 full rows read x and hb in split form, left so by
+    // the launch that made them.
+    const bool use_split = !last && q8_split_usable(rows, dim, hid);
+    char* const xs = reinterpret_cast<char*>(use_split ? m->xsplit.ptr : nullptr);
+    char* const hs = reinterpret_cast<char*>(use_split ? m->hsplit.ptr : nullptr);
+    auto x_out = [&](const float* next_norm) { return next_norm ? Q8SplitOut{xs, next_norm, dim / 32} : Q8SplitOut{}; };
     hip_check(launch_embed_rows(m->f32(m->o_emb), tokens, m->x.ptr, rows, dim, m->vocab, pool->bad_pages.ptr,
-                                m->ss.ptr, s),
+                                m->ss.ptr, use_split ? x_out(m->f32(m->o_rms_att)) : Q8SplitOut{}, s),
               "embed launch");
-    void* const split = rows > 64 ? m->split.ptr : nullptr;
     for (int l = 0; l < m->n_layers; l++) {
         // q, k, v = wq/wk/wv . rms_norm(x, rms_att) in one launch, RoPE on q and
         // k, k and v appended to the pools (:586-617)
@@ -154,24 +162,28 @@ void layers(nitro_model* m, nitro_kvpool* pool, const int32_t* tokens, int rows,
         tqkv.w[2] = m->q8t(m->t_wv, l, kv, dim);
         const int dqkv[3] = {dim, kv, kv};
         rope.layer_off = pool->layer_offset(l);
-        hip_check(launch_q8_qkv(wqkv, m->x.ptr, m->q.ptr, dqkv, rows, dim, last, att, rope, s, tqkv, split),
+        hip_check(launch_q8_qkv(wqkv, m->x.ptr, m->q.ptr, dqkv, rows, dim, last, att, rope, s, tqkv,
+                                Q8Split{xs, {}, nullptr}),
                   "q8_qkv launch");
+        const Q8Norm ffn{m->f32(m->o_rms_ffn) + (size_t)l * dim, m->ss.ptr, parts, rows};
         attend(l);  // attention over the pools -> m->attn (:618-662)
         // x += wo . attn (:663-666)
         hip_check(launch_q8_residual(m->q8(m->o_wo, l, dim, dim), m->attn.ptr, m->x.ptr, m->ss.ptr, rows, dim,
-                                     dim, last, s, m->q8t(m->t_wo, l, dim, dim), split),
+                                     dim, last, s, m->q8t(m->t_wo, l, dim, dim),
+                                     Q8Split{nullptr, use_split ? x_out(ffn.weight) : Q8SplitOut{}, hs}),
                   "q8 wo launch");
         // hb = silu(w1 . xb) * (w3 . xb), xb = rms_norm(x, rms_ffn), one launch (:667-680)
-        const Q8Norm ffn{m->f32(m->o_rms_ffn) + (size_t)l * dim, m->ss.ptr, parts, rows};
         Q8Tiled t13;
         t13.w[0] = m->q8t(m->t_w1, l, hid, dim);
         t13.w[1] = m->q8t(m->t_w3, l, hid, dim);
         hip_check(launch_q8_swiglu(m->q8(m->o_w1, l, hid, dim), m->q8(m->o_w3, l, hid, dim), m->x.ptr,
-                                   m->hb.ptr, rows, dim, hid, last, ffn, s, t13, split),
+                                   m->hb.ptr, rows, dim, hid, last, ffn, s, t13,
+                                   Q8Split{xs, Q8SplitOut{hs, nullptr, hid / 32}, nullptr}),
                   "q8_swiglu launch");
         // x += w2 . hb (:682-684)
         hip_check(launch_q8_residual(m->q8(m->o_w2, l, dim, hid), m->hb.ptr, m->x.ptr, m->ss.ptr, rows, hid,
-                                     dim, last, s, m->q8t(m->t_w2, l, dim, hid), split),
+                                     dim, last, s, m->q8t(m->t_w2, l, dim, hid),
+                                     Q8Split{hs, use_split && l + 1 < m->n_layers ? x_out(att.weight + dim) : Q8SplitOut{}, nullptr}),
                   "q8 w2 launch");
     }
 }

@@ -15,6 +15,7 @@
 #include <cmath>
 
 #include "device_pool.hpp"
+#include "q8_group.hpp"
 
 namespace nitro {
 namespace {
@@ -39,7 +40,7 @@ __global__ __launch_bounds__(ROW_THREADS) void embed_rows_kernel(const float* __
                                                                  const int32_t* __restrict__ tokens,
                                                                  float* __restrict__ x, int dim,
                                                                  int vocab, int32_t* bad_tokens,
-                                                                 float* __restrict__ ss) {
+                                                                 float* __restrict__ ss, Q8SplitOut split) {
     __shared__ float red[ROW_THREADS / 64];
     const int r = blockIdx.x;
     int t = tokens[r];
@@ -54,6 +55,18 @@ __global__ __launch_bounds__(ROW_THREADS) void embed_rows_kernel(const float* __
         const float4 v = src[i];
         dst[i] = v;
         sq = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, sq))));
+        if (split.planes) {  // uniform
+            const float4 w = reinterpret_cast<const float4*>(split.weight)[i];
+            const float p[4] = {v.x * w.x, v.y * w.y, v.z * w.z, v.w * w.w};
+            uint16_t part[3][4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) split_parts(p[j], part[0][j], part[1][j], part[2][j]);
+            char* d = split.planes + split_at(r, 4 * i, split.nb);
+#pragma unroll
+            for (int q = 0; q < 3; q++)
+                *reinterpret_cast<uint2*>(d + 1024 * q) = make_uint2(part[q][0] | (uint32_t)part[q][1] << 16,
+                                                                     part[q][2] | (uint32_t)part[q][3] << 16);
+        }
     }
     if (ss) {  // uniform
         sq = block_sum(sq, red);
@@ -446,9 +459,9 @@ __global__ __launch_bounds__(64 * F32M_WAVES) void f32_matmul_mfma_kernel(const 
 }  // namespace
 
 hipError_t launch_embed_rows(const float* table, const int32_t* tokens, float* x, int rows, int dim,
-                             int vocab, int32_t* bad_tokens, float* ss, hipStream_t stream) {
+                             int vocab, int32_t* bad_tokens, float* ss, const Q8SplitOut& split, hipStream_t stream) {
     hipLaunchKernelGGL(embed_rows_kernel, dim3(rows), dim3(ROW_THREADS), 0, stream, table, tokens, x,
-                       dim, vocab, bad_tokens, ss);
+                       dim, vocab, bad_tokens, ss, split);
     return hipGetLastError();
 }
 

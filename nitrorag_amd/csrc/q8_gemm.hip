@@ -22,7 +22,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // weight row l%16, k = 8*(l/16) .. +8 of a 32-k block).
 //  - x, as the exact sum of three bf16 parts: a wave alone reads its rows, so
 //    they go to registers and not through LDS.  PRE: the parts were written
-//    once by q8_split_kernel in operand order, 1 KB per load instruction;
+//    in operand order where x was made, 1 KB per load instruction;
 //    otherwise the wave splits its rows itself, once per 16 NT weight rows.
 //    (Split per 16 weight rows, as q8_mma_kernel does, and read again from L2
 //    each time, x cost more than the products.)
@@ -53,9 +53,10 @@ __device__ __forceinline__ int w_at(int row, int c) { return row * 32 + ((c ^ (r
 
 template <Q8Epilogue EPI, bool TILED, bool PRE, int GEMM_NT>
 __global__ __launch_bounds__(64 * GEMM_WAVES, GEMM_NT == 8 ? 2 : 3) void q8_gemm_kernel(Q8Group grp, const void* __restrict__ xin,
-                                                                     int batch, int n, int col_tiles, Q8Resid resid,
-                                                                     Q8Rope rope) {
+                                                                     int batch, int n, int col_tiles, Q8Norm nm, Q8Resid resid,
+                                                                     Q8SplitOut out, Q8Rope rope) {
     constexpr int GEMM_BN = 16 * GEMM_NT;
+    constexpr bool NORM = EPI == Q8Epilogue::SwiGlu || EPI == Q8Epilogue::Rope;
     constexpr bool SWIGLU = EPI == Q8Epilogue::SwiGlu;
     constexpr int MROWS = SWIGLU ? GEMM_BN / 2 : GEMM_BN;  // rows of a member per workgroup
     __shared__ __attribute__((aligned(16))) uint16_t wlds[2][GEMM_BN * 32];
@@ -267,6 +268,12 @@ __global__ __launch_bounds__(64 * GEMM_WAVES, GEMM_NT == 8 ? 2 : 3) void q8_gemm
     load_w(wa, 1);
     stage_w(wb, 0);
     load_w(wb, 2);
+    float inv = 1.0f;  // 1/rms of batch row b0 + lane % 32
+    if constexpr (NORM) {  // lanes l and l + 32 add a row's even and odd partials
+        float ss = partial_sum_unbranched<16>(nm, min(b0 + (lane & 31), batch - 1), lane >> 5, 2);
+        ss += __shfl_xor(ss, 32);
+        inv = inv_rms(ss, n);
+    }
     static_assert(GEMM_FLUSH % 2 == 0, "blocks in pairs");
     int blk = 0;
     for (int end = GEMM_FLUSH; end <= nb; end += GEMM_FLUSH) {
@@ -301,18 +308,49 @@ __global__ __launch_bounds__(64 * GEMM_WAVES, GEMM_NT == 8 ? 2 : 3) void q8_gemm
 #pragma unroll
     for (int m = 0; m < GEMM_MT; m++) {
         const int bm = b0 + 16 * m + 4 * lg;
+        if constexpr (NORM) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float f = __shfl(inv, 16 * m + 4 * lg + i);
+#pragma unroll
+                for (int t = 0; t < GEMM_NT; t++) acc[m][t][i] *= f;
+            }
+        }
+        // The wave's 16 x COLS outputs of tile m through LDS (rows 4 floats
+        // apart in banks) into split form, one run of 8 columns per lane.
+        constexpr int COLS = SWIGLU ? GEMM_BN / 2 : GEMM_BN;
+        float* const rows = reinterpret_cast<float*>(&sums[wave][0][0]);
+        static_assert(16 * (COLS + 4) <= GEMM_MT * GEMM_NT * 256, "the outputs fit the wave's sums");
+        auto write_split = [&]() __attribute__((always_inline)) {
+            if (b0 + 16 * m >= batch) return;  // wave-uniform
+#pragma unroll
+            for (int j = 0; j < COLS / 32; j++) {
+                const int k = row0 + 32 * j + 8 * lg;
+                if (row0 + 32 * j >= d) break;  // uniform (d is a multiple of 32)
+                const float* src = rows + lr * (COLS + 4) + 32 * j + 8 * lg;
+                float v[8];
+#pragma unroll
+                for (int i = 0; i < 8; i++) v[i] = out.weight ? src[i] * out.weight[k + i] : src[i];
+                bf16x8 p[3];
+                split3(v, p[0], p[1], p[2]);
+                char* dst = out.planes + split_at(b0 + 16 * m + lr, k, out.nb);
+#pragma unroll
+                for (int i = 0; i < 3; i++) *reinterpret_cast<bf16x8*>(dst + 1024 * i) = p[i];
+            }
+        };
         if constexpr (SWIGLU) {
             // the first half of the tiles are w1's rows, the second the same rows of w3
 #pragma unroll
             for (int t = 0; t < GEMM_NT / 2; t++) {
-                const int row = row0 + 16 * t + lr;
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     float h = acc[m][t][i];
                     h *= 1.0f / (1.0f + expf(-h));
-                    if (bm + i < batch && row < d) grp.out[0][(size_t)(bm + i) * d + row] = h * acc[m][t + GEMM_NT / 2][i];
+                    h *= acc[m][t + GEMM_NT / 2][i];
+                    rows[(4 * lg + i) * (COLS + 4) + 16 * t + lr] = h;
                 }
             }
+            write_split();
         } else if constexpr (EPI == Q8Epilogue::Residual) {
             // x += product; the squares of the new entries are added over each
             // 16-row tile's 16 lanes (one partial per batch row and tile)
@@ -327,12 +365,14 @@ __global__ __launch_bounds__(64 * GEMM_WAVES, GEMM_NT == 8 ? 2 : 3) void q8_gemm
                     const float v = xv[i] + acc[m][t][i];
                     const bool ok = bm + i < batch && row < d;
                     if (ok) grp.out[0][(size_t)(bm + i) * d + row] = v;
+                    rows[(4 * lg + i) * (COLS + 4) + 16 * t + lr] = v;
                     float sq = ok ? v * v : 0.0f;
 #pragma unroll
                     for (int msk = 8; msk > 0; msk >>= 1) sq += __shfl_xor(sq, msk, 16);
                     if (lr == 0 && ok) resid.ss[(size_t)(row >> 4) * resid.ss_stride + bm + i] = sq;
                 }
             }
+            if (out.planes) write_split();  // uniform
         } else if constexpr (EPI == Q8Epilogue::Rope) {
             // RoPE pairs are adjacent weight rows, so adjacent lanes
 #pragma unroll
@@ -372,44 +412,25 @@ __global__ __launch_bounds__(64 * GEMM_WAVES, GEMM_NT == 8 ? 2 : 3) void q8_gemm
     }
 }
 
-// Activations split once for q8_gemm_kernel (the layout at Q8_SPLIT_BYTES):
-// workgroup (tile, group) takes 16 rows x 16 blocks, wave w blocks w, w + 4, ..;
-// a lane reads its run of 8 k as floats (NORM: rms_norm applied) and writes it
-// as three bf16 runs.
-template <bool NORM>
+// fp32 activations to split form: workgroup (tile, group) takes 16 rows x 16
+// blocks, wave w blocks w, w + 4, ..; a lane reads a run of 8 k and writes it as
+// three bf16 runs.
 __global__ __launch_bounds__(256) void q8_split_kernel(const float* __restrict__ x, char* __restrict__ out, int rows,
-                                                       int n, Q8Norm nm) {
-    __shared__ float part[16][16];
+                                                       int n) {
     const int nb = n / Q8_BLOCK;
-    const int tile = blockIdx.x, lane = threadIdx.x & 63;
-    const int row = min(tile * 16 + (lane & 15), rows - 1);
-    float inv = 1.0f;
-    if constexpr (NORM) {
-        part[threadIdx.x >> 4][lane & 15] = partial_sum_unbranched<4>(nm, row, threadIdx.x >> 4, 16);
-        __syncthreads();
-        float s = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 16; i++) s += part[i][lane & 15];
-        inv = inv_rms(s, n);
-    }
+    const int lane = threadIdx.x & 63;
+    const int row = blockIdx.x * 16 + (lane & 15);
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const int blk = blockIdx.y * 16 + 4 * i + (threadIdx.x >> 6);
         if (blk >= nb) break;  // wave-uniform
         const int k = blk * Q8_BLOCK + 8 * (lane >> 4);
-        const float4 a = reinterpret_cast<const float4*>(x + (size_t)row * n + k)[0];
-        const float4 b = reinterpret_cast<const float4*>(x + (size_t)row * n + k)[1];
-        float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-        if constexpr (NORM) {
-            const float4 wa = reinterpret_cast<const float4*>(nm.weight + k)[0];
-            const float4 wb = reinterpret_cast<const float4*>(nm.weight + k)[1];
-            const float w[8] = {wa.x, wa.y, wa.z, wa.w, wb.x, wb.y, wb.z, wb.w};
-#pragma unroll
-            for (int j = 0; j < 8; j++) v[j] = w[j] * (inv * v[j]);
-        }
+        const float4* src = reinterpret_cast<const float4*>(x + (size_t)min(row, rows - 1) * n + k);
+        const float4 a = src[0], b = src[1];
+        const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
         bf16x8 p[3];
         split3(v, p[0], p[1], p[2]);
-        char* dst = out + ((size_t)tile * nb + blk) * Q8_SPLIT_BYTES + lane * 16;
+        char* dst = out + split_at(row, k, nb);
 #pragma unroll
         for (int j = 0; j < 3; j++) *reinterpret_cast<bf16x8*>(dst + 1024 * j) = p[j];
     }
@@ -417,26 +438,18 @@ __global__ __launch_bounds__(256) void q8_split_kernel(const float* __restrict__
 
 template <Q8Epilogue EPI, bool PRE, int NT>
 void launch(bool tiled, dim3 grid, hipStream_t stream, const Q8Group& grp, const void* x, int batch, int n, int cols,
-            const Q8Resid& resid, const Q8Rope& rope) {
+            const Q8Norm& nm, const Q8Resid& resid, const Q8SplitOut& out, const Q8Rope& rope) {
     if (tiled)
         hipLaunchKernelGGL((q8_gemm_kernel<EPI, true, PRE, NT>), grid, dim3(64 * GEMM_WAVES), 0, stream, grp, x, batch,
-                           n, cols, resid, rope);
+                           n, cols, nm, resid, out, rope);
     else
         hipLaunchKernelGGL((q8_gemm_kernel<EPI, false, PRE, NT>), grid, dim3(64 * GEMM_WAVES), 0, stream, grp, x, batch,
-                           n, cols, resid, rope);
+                           n, cols, nm, resid, out, rope);
 }
 
 }  // namespace
 
-void launch_q8_split(const float* x, void* split, int rows, int n, const Q8Norm& nm, hipStream_t stream) {
-    const dim3 grid((unsigned)((rows + 15) / 16), (unsigned)((n / Q8_BLOCK + 15) / 16));
-    if (nm.weight)
-        hipLaunchKernelGGL(q8_split_kernel<true>, grid, dim3(256), 0, stream, x, static_cast<char*>(split), rows, n, nm);
-    else
-        hipLaunchKernelGGL(q8_split_kernel<false>, grid, dim3(256), 0, stream, x, static_cast<char*>(split), rows, n, nm);
-}
-
-bool launch_q8_gemm(Q8Epilogue epilogue, const Q8Group& grp, const float* x, void* split, int batch, int n,
+bool launch_q8_gemm(Q8Epilogue epilogue, const Q8Group& grp, const float* x, const Q8Split& split, int batch, int n,
                     const Q8Norm& nm, const Q8Resid& resid, const Q8Rope& rope, hipStream_t stream) {
     const int members = epilogue == Q8Epilogue::Rope ? 3 : epilogue == Q8Epilogue::SwiGlu ? 2 : 1;
     bool tiled = true;
@@ -446,7 +459,9 @@ bool launch_q8_gemm(Q8Epilogue epilogue, const Q8Group& grp, const float* x, voi
         dmax = std::max(dmax, grp.d[m]);
     }
     if (q8_tiled_bytes(dmax, n) >= (1ull << 32) || q8_split_bytes(batch, n) >= (1ull << 32)) return false;
-    if (epilogue != Q8Epilogue::Store && !split) return false;
+    const bool pre = epilogue != Q8Epilogue::Store;
+    if (pre && !split.in && (!split.scratch || nm.weight)) return false;
+    if (epilogue == Q8Epilogue::SwiGlu && !split.out.planes) return false;
     auto columns = [&](int bn) {  // column tiles of bn weight rows
         int c = 0;
         for (int m = 0; m < members; m++) c += (grp.d[m] + bn - 1) / bn;
@@ -464,7 +479,7 @@ bool launch_q8_gemm(Q8Epilogue epilogue, const Q8Group& grp, const float* x, voi
     const long long wide = panels * columns(128), slim = panels * columns(64);
     const long long wide_rounds = (wide + 2 * CUS - 1) / (2 * CUS), slim_rounds = (slim + 3 * CUS - 1) / (3 * CUS);
     const double wide_fill = (double)wide / (wide_rounds * 2 * CUS), slim_fill = (double)slim / (slim_rounds * 3 * CUS);
-    const bool narrow = slim_fill * (split ? 1.0 : 0.75) > wide_fill;
+    const bool narrow = slim_fill * (pre ? 1.0 : 0.75) > wide_fill;
     const long long wgs = narrow ? slim : wide;
     // A round takes about 1 us per block (1.3 with 128 rows) at any size, the
     // small-batch kernel rows x outputs x n / 26.5e6 us, so this kernel pays
@@ -477,14 +492,21 @@ bool launch_q8_gemm(Q8Epilogue epilogue, const Q8Group& grp, const float* x, voi
     if (wgs > (1ll << 30) || outputs < (narrow ? 830e3 * slim_rounds : 1080e3 * wide_rounds)) return false;
     const int cols = columns(narrow ? 64 : 128);
     const dim3 grid((unsigned)wgs);
-    if (split) launch_q8_split(x, split, batch, n, nm, stream);
+    const void* in = x;
+    if (pre && split.in) {
+        in = split.in;
+    } else if (pre) {
+        hipLaunchKernelGGL(q8_split_kernel, dim3((unsigned)((batch + 15) / 16), (unsigned)((n / Q8_BLOCK + 15) / 16)),
+                           dim3(256), 0, stream, x, static_cast<char*>(split.scratch), batch, n);
+        in = split.scratch;
+    }
     const auto run = [&](auto nt) {
         constexpr int NT = decltype(nt)::value;
         switch (epilogue) {
-            case Q8Epilogue::Store: launch<Q8Epilogue::Store, false, NT>(tiled, grid, stream, grp, x, batch, n, cols, resid, rope); break;
-            case Q8Epilogue::Residual: launch<Q8Epilogue::Residual, true, NT>(tiled, grid, stream, grp, split, batch, n, cols, resid, rope); break;
-            case Q8Epilogue::SwiGlu: launch<Q8Epilogue::SwiGlu, true, NT>(tiled, grid, stream, grp, split, batch, n, cols, resid, rope); break;
-            case Q8Epilogue::Rope: launch<Q8Epilogue::Rope, true, NT>(tiled, grid, stream, grp, split, batch, n, cols, resid, rope); break;
+            case Q8Epilogue::Store: launch<Q8Epilogue::Store, false, NT>(tiled, grid, stream, grp, in, batch, n, cols, nm, resid, split.out, rope); break;
+            case Q8Epilogue::Residual: launch<Q8Epilogue::Residual, true, NT>(tiled, grid, stream, grp, in, batch, n, cols, nm, resid, split.out, rope); break;
+            case Q8Epilogue::SwiGlu: launch<Q8Epilogue::SwiGlu, true, NT>(tiled, grid, stream, grp, in, batch, n, cols, nm, resid, split.out, rope); break;
+            case Q8Epilogue::Rope: launch<Q8Epilogue::Rope, true, NT>(tiled, grid, stream, grp, in, batch, n, cols, nm, resid, split.out, rope); break;
         }
     };
     if (narrow)

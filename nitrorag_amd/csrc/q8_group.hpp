@@ -6,6 +6,7 @@
 
 #include <cstdint>
 
+#include "bf16_split.hpp"
 #include "device_pool.hpp"
 
 namespace nitro {
@@ -72,13 +73,28 @@ __device__ __forceinline__ float2 rotate_pair(const Q8Rope& rp, int pos, int fea
     return make_float2(x * c - y * sn, x * sn + y * c);
 }
 
+// Byte offset of (row, column k)'s part 0 in split form (part p: + 1024 p).
+__device__ __forceinline__ size_t split_at(int row, int k, int nb) {
+    return ((size_t)(row >> 4) * nb + (k >> 5)) * Q8_SPLIT_BYTES + ((row & 15) + 16 * ((k >> 3) & 3)) * 16 + (k & 7) * 2;
+}
+
+// One value of a product's output in split form.
+__device__ __forceinline__ void store_split(const Q8SplitOut& o, int row, int k, float v) {
+    if (o.weight) v *= o.weight[k];
+    uint16_t hi, mid, lo;
+    split_parts(v, hi, mid, lo);
+    char* dst = o.planes + split_at(row, k, o.nb);
+    *reinterpret_cast<uint16_t*>(dst) = hi;
+    *reinterpret_cast<uint16_t*>(dst + 1024) = mid;
+    *reinterpret_cast<uint16_t*>(dst + 2048) = lo;
+}
+
 // What a large product does with its sums.
 enum class Q8Epilogue { Store, Residual, SwiGlu, Rope };
 
 // The large-batch product (q8_gemm.hip): true if launched, false where the
-// shapes are not its own (the caller takes another kernel).  split: workspace
-// of q8_split_bytes(batch, n) for the split activations, or null.
-bool launch_q8_gemm(Q8Epilogue epilogue, const Q8Group& grp, const float* x, void* split, int batch, int n,
+// shapes are not its own (the caller takes another kernel).
+bool launch_q8_gemm(Q8Epilogue epilogue, const Q8Group& grp, const float* x, const Q8Split& split, int batch, int n,
                     const Q8Norm& nm, const Q8Resid& resid, const Q8Rope& rope, hipStream_t stream);
 
 }  // namespace nitro

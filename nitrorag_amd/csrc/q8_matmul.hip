@@ -626,7 +626,8 @@ __global__ __launch_bounds__(64 * GEMV_WAVES) void q8_gemv_kernel(Q8Group grp, c
 // and call this together; they add their squares into partial p of row b.
 template <int NMAT, bool SWIGLU, bool RESID, bool ROPE>
 __device__ __forceinline__ void store_row_sums(const Q8Group& grp, const Q8Resid& resid, const Q8Rope& rope, int b,
-                                               int row, const float (&sum)[NMAT], const float (&pair)[2]) {
+                                               int row, const float (&sum)[NMAT], const float (&pair)[2],
+                                               const Q8SplitOut& out = Q8SplitOut{}) {
     if constexpr (ROPE) {
         const RopeRow rp = rope_row(rope, b);
         const bool odd = row & 1;
@@ -652,6 +653,7 @@ __device__ __forceinline__ void store_row_sums(const Q8Group& grp, const Q8Resid
             const float v = *xe + sum[0];
             *xe = v;
             ssq = v * v;
+            if (out.planes) store_split(out, b, row, v);
         }
 #pragma unroll
         for (int msk = 8; msk > 0; msk >>= 1) ssq += __shfl_xor(ssq, msk, 16);
@@ -660,7 +662,10 @@ __device__ __forceinline__ void store_row_sums(const Q8Group& grp, const Q8Resid
         if (row < grp.d[0]) {
             float h = sum[0];
             h *= 1.0f / (1.0f + expf(-h));
-            grp.out[0][(size_t)b * grp.d[0] + row] = h * sum[1];
+            if (out.planes)
+                store_split(out, b, row, h * sum[1]);
+            else
+                grp.out[0][(size_t)b * grp.d[0] + row] = h * sum[1];
         }
     } else {
 #pragma unroll
@@ -1141,6 +1146,14 @@ __global__ __launch_bounds__(64 * flat_waves<RESID>()) void q8_flat_kernel(Q8Gro
 // holding out[batch 4*(l/16) + j][row l%16] and every lane scales by the
 // scale of its own row.
 //
+// PRE (a model's launches but wo): x arrives in split form (Q8Split), written
+// where it was made, so the loop neither splits nor normalises it and loads 1
+// KB per instruction; the norm weights are in it and 1/rms scales the sums.
+// (The split and norm of x were two thirds of the loop's VALU work: 32 rows,
+// 110M-parameter shapes, w1/w3 5.6 -> 5.0 us, wq/wk/wv 7.2 -> 5.6, wo and w2
+// 6.4 -> 5.0 on average; 8 rows, 4096 x 11008, w1/w3 41.6 -> 30.9, wq/wk/wv
+// 19.2 -> 16.6.)
+//
 // A workgroup owns 16 rows of each group member and 16 or 32 batch rows (BT
 // tiles of 16; larger batches add workgroups along y); MMA_WAVES waves take the rows' blocks U at a time,
 // round-robin.  A wave's rounds are pipelined: it loads a round's x (an L2
@@ -1177,21 +1190,22 @@ constexpr int MMA_MAX_BT = 2;       // batch tiles per workgroup (more rows: mor
 constexpr int MMA_NORM_MAX_N = 8192;  // rms weights staged in LDS (larger n: the fp32 kernel)
 
 // One round of a wave: weights and x of U blocks.
-template <int NMAT, int BT, int U>
+template <int NMAT, int BT, int U, bool PRE>
 struct MmaRound {
     uint32_t q[U][NMAT][2];
     float scale[U][NMAT];
-    float x[BT][U][8];
+    u32x4 x[BT][U][PRE ? 3 : 2];  // PRE: hi, mid, lo; else 8 floats
 };
 
-template <int NMAT, int BT, bool TILED, bool SWIGLU, bool NORM, bool RESID, bool ROPE>
-__global__ __launch_bounds__(64 * MMA_WAVES) void q8_mma_kernel(Q8Group grp, const float* __restrict__ x, int batch,
-                                                                int n, Q8Norm nm, Q8Resid resid, Q8Rope rope) {
+template <int NMAT, int BT, bool TILED, bool PRE, bool SWIGLU, bool NORM, bool RESID, bool ROPE>
+__global__ __launch_bounds__(64 * MMA_WAVES) void q8_mma_kernel(Q8Group grp, const void* __restrict__ xin,
+                                                                int batch, int n, Q8Norm nm, Q8Resid resid,
+                                                                Q8SplitOut out, Q8Rope rope) {
     constexpr int U = mma_unroll<NMAT, BT>();
     constexpr int STRIDE = MMA_WAVES * U;  // blocks per round of the workgroup
     __shared__ float red[MMA_WAVES][NMAT][16 * MMA_TILE_STRIDE];
     __shared__ float norm_s[NORM ? MMA_WAVES * 64 : 1];
-    __shared__ float norm_w[NORM ? MMA_NORM_MAX_N : 1];
+    __shared__ float norm_w[NORM && !PRE ? MMA_NORM_MAX_N : 1];
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int r = lane & 15;
@@ -1222,9 +1236,19 @@ __global__ __launch_bounds__(64 * MMA_WAVES) void q8_mma_kernel(Q8Group grp, con
             soff[m] = row;
         }
     }
-    uint32_t xrow[BT];
+    // x: byte offset of this lane's run of block 0 (PRE: batch tiles clamped; in a
+    // tile of up to 8 rows, lanes of rows 8..15 reread rows 0..7, so that half
+    // the lines are read)
+    const char* const xb = static_cast<const char*>(xin);
+    uint32_t xoff[BT];
 #pragma unroll
-    for (int t = 0; t < BT; t++) xrow[t] = (uint32_t)min(b0 + t * 16 + r, batch - 1) * n + 8 * g;
+    for (int t = 0; t < BT; t++)
+        if constexpr (PRE)
+            xoff[t] = (uint32_t)min(b0 / 16 + t, (batch - 1) / 16) * nb * Q8_SPLIT_BYTES +
+                      16 * (batch - (b0 + t * 16) <= 8 ? lane & ~8 : lane);
+        else
+            xoff[t] = ((uint32_t)min(b0 + t * 16 + r, batch - 1) * n + 8 * g) * 4;
+    constexpr uint32_t XSTEP = PRE ? Q8_SPLIT_BYTES : Q8_BLOCK * 4;
     f32x4 acc[NMAT][BT];
 #pragma unroll
     for (int m = 0; m < NMAT; m++)
@@ -1232,7 +1256,7 @@ __global__ __launch_bounds__(64 * MMA_WAVES) void q8_mma_kernel(Q8Group grp, con
         for (int t = 0; t < BT; t++) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 
-    using Round = MmaRound<NMAT, BT, U>;
+    using Round = MmaRound<NMAT, BT, U, PRE>;
     auto load_round = [&](Round& R, int base) {
 #pragma unroll
         for (int u = 0; u < U; u++) {
@@ -1246,12 +1270,10 @@ __global__ __launch_bounds__(64 * MMA_WAVES) void q8_mma_kernel(Q8Group grp, con
                 R.scale[u][m] = *reinterpret_cast<const float*>(wbase[m] + (soff[m] + (uint32_t)blk * BSTEP));
             }
 #pragma unroll
-            for (int t = 0; t < BT; t++) {
-                const float4 a = *reinterpret_cast<const float4*>(x + (xrow[t] + blk * Q8_BLOCK));
-                const float4 c = *reinterpret_cast<const float4*>(x + (xrow[t] + blk * Q8_BLOCK + 4));
-                R.x[t][u][0] = a.x, R.x[t][u][1] = a.y, R.x[t][u][2] = a.z, R.x[t][u][3] = a.w;
-                R.x[t][u][4] = c.x, R.x[t][u][5] = c.y, R.x[t][u][6] = c.z, R.x[t][u][7] = c.w;
-            }
+            for (int t = 0; t < BT; t++)
+#pragma unroll
+                for (int p = 0; p < (PRE ? 3 : 2); p++)
+                    R.x[t][u][p] = *reinterpret_cast<const u32x4*>(xb + (xoff[t] + (uint32_t)blk * XSTEP + (PRE ? 1024 : 16) * p));
         }
     };
     // per block: its weights as bf16, then per batch tile the split x and
@@ -1264,17 +1286,23 @@ __global__ __launch_bounds__(64 * MMA_WAVES) void q8_mma_kernel(Q8Group grp, con
             for (int m = 0; m < NMAT; m++) wb[m] = q8_bf16(R.q[u][m][0], R.q[u][m][1]);
 #pragma unroll
             for (int t = 0; t < BT; t++) {
-                float v[8];
-#pragma unroll
-                for (int i = 0; i < 8; i++) v[i] = R.x[t][u][i];
-                if constexpr (NORM) {
-                    const float inv = norm_s[t * 16 + r];
-                    const int k0 = min(base + u, nb - 1) * Q8_BLOCK + 8 * g;
-#pragma unroll
-                    for (int i = 0; i < 8; i++) v[i] = norm_w[k0 + i] * (inv * v[i]);
-                }
                 bf16x8 xh, xm, xl;
-                split3(v, xh, xm, xl);
+                if constexpr (PRE) {
+                    xh = __builtin_bit_cast(bf16x8, R.x[t][u][0]);
+                    xm = __builtin_bit_cast(bf16x8, R.x[t][u][1]);
+                    xl = __builtin_bit_cast(bf16x8, R.x[t][u][2]);
+                } else {
+                    float v[8];
+#pragma unroll
+                    for (int i = 0; i < 8; i++) v[i] = __uint_as_float(R.x[t][u][i >> 2][i & 3]);
+                    if constexpr (NORM) {
+                        const float inv = norm_s[t * 16 + r];
+                        const int k0 = min(base + u, nb - 1) * Q8_BLOCK + 8 * g;
+#pragma unroll
+                        for (int i = 0; i < 8; i++) v[i] = norm_w[k0 + i] * (inv * v[i]);
+                    }
+                    split3(v, xh, xm, xl);
+                }
                 f32x4 sm[NMAT];
 #pragma unroll
                 for (int m = 0; m < NMAT; m++) sm[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xl, wb[m], zero, 0, 0, 0);
@@ -1298,8 +1326,18 @@ __global__ __launch_bounds__(64 * MMA_WAVES) void q8_mma_kernel(Q8Group grp, con
     // before the current round is computed.
     Round ra, rb;
     int base = wave * U;
+    if constexpr (NORM && PRE) {
+        // thread (row j = tid % 64, class c = tid / 64) adds partials c, c + 8, ...;
+        // the epilogue adds row j's class sums in class order.  (The partials'
+        // loads go out before the first round's, which stay in flight.)
+        const int j = threadIdx.x & 63, c = threadIdx.x >> 6;
+        const int prow = min(b0 + min(j, 16 * BT - 1), batch - 1);
+        const float ps = nm.nparts <= 4 * MMA_WAVES ? partial_sum_unbranched<4>(nm, prow, c, MMA_WAVES)
+                                                    : partial_sum_unbranched<16>(nm, prow, c, MMA_WAVES);
+        norm_s[c * 64 + j] = ps;
+    }
     if (base < nb) load_round(ra, base);  // in flight while the norm prologue runs
-    if constexpr (NORM) {
+    if constexpr (NORM && !PRE) {
         // thread (row j = tid % 64, class c = tid / 64) adds partials c, c + 16, ...;
         // row j's class sums are then added in class order: norm_s[j] = inv_rms
         // The rms weights' loads and the partials' loads go out together
@@ -1371,7 +1409,17 @@ __global__ __launch_bounds__(64 * MMA_WAVES) void q8_mma_kernel(Q8Group grp, con
                     pair[0] = sums[0][threadIdx.x ^ 1];
                     pair[1] = sums[1][threadIdx.x ^ 1];
                 }
-                store_row_sums<NMAT, SWIGLU, RESID, ROPE>(grp, resid, rope, b, row0 + i, sum, pair);
+                if constexpr (NORM && PRE) {
+                    float ss = 0.0f;
+#pragma unroll
+                    for (int c = 0; c < MMA_WAVES; c++) ss += norm_s[c * 64 + t * 16 + bl];
+                    const float inv = inv_rms(ss, n);
+#pragma unroll
+                    for (int m = 0; m < NMAT; m++) sum[m] *= inv;
+                    pair[0] *= inv;
+                    pair[1] *= inv;
+                }
+                store_row_sums<NMAT, SWIGLU, RESID, ROPE>(grp, resid, rope, b, row0 + i, sum, pair, out);
             }
         }
     }
@@ -1461,9 +1509,9 @@ void launch_gemv(const Q8Group& grp, const float* x, int n, int dmax, const Q8No
                        rs, rp);
 }
 
-template <int NMAT, bool TILED, bool SWIGLU, bool NORM, bool RESID, bool ROPE>
-void launch_mma(const Q8Group& grp, const float* x, int batch, int n, int dmax, const Q8Norm& nm, const Q8Resid& rs,
-                const Q8Rope& rp, hipStream_t stream) {
+template <int NMAT, bool TILED, bool PRE, bool SWIGLU, bool NORM, bool RESID, bool ROPE>
+void launch_mma(const Q8Group& grp, const void* x, int batch, int n, int dmax, const Q8Norm& nm, const Q8Resid& rs,
+                const Q8SplitOut& out, const Q8Rope& rp, hipStream_t stream) {
     const dim3 block(64 * MMA_WAVES);
     const unsigned tiles = (unsigned)((dmax + 15) / 16);
     // (three members with two batch tiles would exceed the registers)
@@ -1475,12 +1523,12 @@ void launch_mma(const Q8Group& grp, const float* x, int batch, int n, int dmax, 
     // product at batch 32 (256 tiles) took 32.6 us against 25.2 with two.
     const unsigned btiles = (unsigned)((batch + 15) / 16);
     if (BT == 1 || btiles == 1 || (long long)tiles * btiles <= device_cus()) {
-        hipLaunchKernelGGL((q8_mma_kernel<NMAT, 1, TILED, SWIGLU, NORM, RESID, ROPE>), dim3(tiles, btiles), block,
-                           0, stream, grp, x, batch, n, nm, rs, rp);
+        hipLaunchKernelGGL((q8_mma_kernel<NMAT, 1, TILED, PRE, SWIGLU, NORM, RESID, ROPE>), dim3(tiles, btiles), block,
+                           0, stream, grp, x, batch, n, nm, rs, out, rp);
     } else {
         const dim3 g2(tiles, (unsigned)((batch + 16 * BT - 1) / (16 * BT)));
-        hipLaunchKernelGGL((q8_mma_kernel<NMAT, BT, TILED, SWIGLU, NORM, RESID, ROPE>), g2, block, 0, stream, grp, x,
-                           batch, n, nm, rs, rp);
+        hipLaunchKernelGGL((q8_mma_kernel<NMAT, BT, TILED, PRE, SWIGLU, NORM, RESID, ROPE>), g2, block, 0, stream, grp, x,
+                           batch, n, nm, rs, out, rp);
     }
 }
 
@@ -1508,7 +1556,7 @@ __global__ __launch_bounds__(64) void q8_tile_kernel(const uint8_t* __restrict__
 
 template <int NMAT, bool SWIGLU, bool NORM, bool RESID, bool ROPE = false>
 void launch_group(const Q8Group& grp, const float* x, int batch, int n, int dmax, bool last, const Q8Norm& nm,
-                  const Q8Resid& rs, hipStream_t stream, const Q8Rope& rp = Q8Rope{}, void* split = nullptr) {
+                  const Q8Resid& rs, hipStream_t stream, const Q8Rope& rp = Q8Rope{}, const Q8Split& split = Q8Split{}) {
     const dim3 grid((unsigned)((dmax + 15) / 16),
                     (unsigned)((batch + 16 * Q8_MAX_BTILES - 1) / (16 * Q8_MAX_BTILES)));
     const dim3 block(64 * Q8_WAVES);
@@ -1530,14 +1578,21 @@ void launch_group(const Q8Group& grp, const float* x, int batch, int n, int dmax
     if (use_mma() && launch_q8_gemm(EPI, grp, x, split, batch, n, nm, rs, rp, stream)) return;
     // the bf16 kernel addresses weights and x with 32-bit offsets
     const bool mma_fits = q8_tiled_bytes(dmax, n) < (1ull << 32) && (size_t)batch * n < (1ull << 32) &&
-                          (!NORM || n <= MMA_NORM_MAX_N);
+                          (!NORM || split.in || n <= MMA_NORM_MAX_N);
     if (use_mma() && mma_fits) {
         bool tiled = true;
         for (int m = 0; m < NMAT; m++) tiled = tiled && grp.wt[m] != nullptr;
+        // (a model hands on split activations only where it holds the tile layout)
+        if constexpr (NORM || RESID)
+            if (split.in) {
+                launch_mma<NMAT, true, true, SWIGLU, NORM, RESID, ROPE>(grp, split.in, batch, n, dmax, nm, rs, split.out,
+                                                                        rp, stream);
+                return;
+            }
         if (tiled)
-            launch_mma<NMAT, true, SWIGLU, NORM, RESID, ROPE>(grp, x, batch, n, dmax, nm, rs, rp, stream);
+            launch_mma<NMAT, true, false, SWIGLU, NORM, RESID, ROPE>(grp, x, batch, n, dmax, nm, rs, split.out, rp, stream);
         else
-            launch_mma<NMAT, false, SWIGLU, NORM, RESID, ROPE>(grp, x, batch, n, dmax, nm, rs, rp, stream);
+            launch_mma<NMAT, false, false, SWIGLU, NORM, RESID, ROPE>(grp, x, batch, n, dmax, nm, rs, split.out, rp, stream);
         return;
     }
     hipLaunchKernelGGL((q8_matmul_kernel<NMAT, SWIGLU, NORM, RESID, ROPE>), grid, block, 0, stream, grp, x, batch, n,
@@ -1554,6 +1609,12 @@ hipError_t launch_q8_tile(const void* w, void* tiled, int d, int n, hipStream_t 
     return hipGetLastError();
 }
 
+bool q8_split_usable(size_t rows, size_t dim, size_t hidden) {
+    const size_t wide = std::max(dim, hidden);
+    return use_mma() && rows > (size_t)Q8_GEMV_MAX_BATCH && q8_split_bytes(rows, wide) < (1ull << 32) &&
+           q8_tiled_bytes(wide, wide) < (1ull << 32);
+}
+
 hipError_t launch_q8_matmul(const void* w, const float* x, float* out, int batch, int n, int d,
                             bool last_block_only, hipStream_t stream) {
     Q8Group grp{{static_cast<const uint8_t*>(w), nullptr, nullptr}, {out, nullptr, nullptr}, {d, 0, 0}, {}};
@@ -1562,7 +1623,7 @@ hipError_t launch_q8_matmul(const void* w, const float* x, float* out, int batch
 }
 
 hipError_t launch_q8_residual(const void* w, const float* in, float* x, float* ss, int batch, int n, int d,
-                              bool last_block_only, hipStream_t stream, const void* w_tiled, void* split) {
+                              bool last_block_only, hipStream_t stream, const void* w_tiled, const Q8Split& split) {
     Q8Group grp{{static_cast<const uint8_t*>(w), nullptr, nullptr},
                 {x, nullptr, nullptr},
                 {d, 0, 0},
@@ -1574,7 +1635,7 @@ hipError_t launch_q8_residual(const void* w, const float* in, float* x, float* s
 
 hipError_t launch_q8_qkv(const void* const* w, const float* x, float* out_q, const int* d, int batch, int n,
                          bool last_block_only, const Q8Norm& nm, const Q8Rope& rope, hipStream_t stream,
-                         const Q8Tiled& tiled, void* split) {
+                         const Q8Tiled& tiled, const Q8Split& split) {
     if (!nm.weight || !rope.freq_real || d[1] != d[2] || d[0] % 32 || d[1] % 32) return hipErrorInvalidValue;
     Q8Group grp{};
     for (int m = 0; m < 3; m++) {
@@ -1590,7 +1651,7 @@ hipError_t launch_q8_qkv(const void* const* w, const float* x, float* out_q, con
 
 hipError_t launch_q8_swiglu(const void* w1, const void* w3, const float* x, float* hb, int batch, int n,
                             int hidden, bool last_block_only, const Q8Norm& nm, hipStream_t stream,
-                            const Q8Tiled& tiled, void* split) {
+                            const Q8Tiled& tiled, const Q8Split& split) {
     Q8Group grp{{static_cast<const uint8_t*>(w1), static_cast<const uint8_t*>(w3), nullptr},
                 {hb, nullptr, nullptr},
                 {hidden, hidden, 0},
