@@ -168,7 +168,7 @@ def lib() -> ctypes.CDLL:
 
 def call(name: str, *args) -> None:
     """Calls a status-returning entry point and raises NitroError on failure."""
-    st = getattr(lib(), name)(*args)
+    st = getattr(_lib or lib(), name)(*args)
     if st != OK:
         raise NitroError(st, name, lib().nitro_last_error().decode())
 

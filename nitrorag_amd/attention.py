@@ -19,25 +19,39 @@ import numpy as np
 from . import _native as N
 
 
-def _stream_ptr(stream):
-    import torch
+_torch = None
 
-    if stream is None:
-        stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+
+def _torch_module():
+    global _torch
+    if _torch is None:
+        import torch
+
+        _torch = torch
+    return _torch
+
+
+def _stream_ptr(stream):
+    """The address of a stream, or of torch's current one: its raw handle, without
+    the Stream object that torch.cuda.current_stream() builds."""
+    if stream is not None:
+        return stream.cuda_stream
+    torch = _torch or _torch_module()
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _dev(t, name: str):
-    import torch
-
-    if not isinstance(t, torch.Tensor) or t.device.type != "cuda":
+    torch = _torch or _torch_module()
+    if not isinstance(t, torch.Tensor) or not t.is_cuda:
         raise TypeError(f"{name} must be a GPU tensor")
-    if t.dtype != torch.float32 or not t.is_contiguous():
+    if t.dtype is not torch.float32 or not t.is_contiguous():
         raise TypeError(f"{name} must be contiguous float32")
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 def _host_i32(a) -> np.ndarray:
+    if isinstance(a, np.ndarray) and a.dtype == np.int32:
+        return np.ascontiguousarray(a)
     return np.ascontiguousarray(np.asarray(a, dtype=np.int64).astype(np.int32))
 
 

@@ -553,9 +553,7 @@ void set_device_decode_batch(nitro_kvpool* pool, int batch, int max_pages, const
     require(batch > 0 && max_pages > 0, ERR_INVALID_ARGUMENT, "batch and max_pages must be positive");
     DecodeBatch& d = pool->decode;
     d.batch = 0;
-    d.tables.reserve((size_t)batch * max_pages);
-    d.pos.reserve(batch);
-    d.slots.reserve(batch);
+    d.reserve((size_t)batch * max_pages, batch);
     *device_slots = d.slots.ptr;
     d.positions.assign(positions, positions + batch);
     d.shared_pages = shared_pages;
@@ -693,9 +691,7 @@ int nitro_decode_batch_upload(nitro_kvpool* pool, const int32_t* tables, const i
         DecodeBatch& d = pool->decode;
         const size_t nt = (size_t)batch * max_pages;
         d.batch = 0;  // invalid until the copies are issued
-        d.tables.reserve(nt);
-        d.pos.reserve(batch);
-        d.slots.reserve(batch);
+        d.reserve(nt, batch);
         hipStream_t s = as_stream(stream);
         Staging& st = pool->decode_staging;
         int32_t* h = st.acquire(nt + 2 * (size_t)batch);
@@ -704,9 +700,7 @@ int nitro_decode_batch_upload(nitro_kvpool* pool, const int32_t* tables, const i
         for (int b = 0; b < batch; b++)  // where each row's K/V goes (the fused RoPE/append reads it)
             h[nt + batch + b] = tables[(size_t)b * max_pages + positions[b] / BLOCK_SIZE] * BLOCK_SIZE +
                                 positions[b] % BLOCK_SIZE;
-        st.copy(d.tables.ptr, h, nt, s);
-        st.copy(d.pos.ptr, h + nt, batch, s);
-        st.copy(d.slots.ptr, h + nt + batch, batch, s);
+        st.copy(d.words.ptr, h, nt + 2 * (size_t)batch, s);
         st.finish(s);
         d.positions.assign(positions, positions + batch);
         find_decode_groups(pool, d, tables, positions, batch, max_pages);
@@ -919,22 +913,17 @@ int nitro_prefill_batch_upload(nitro_kvpool* pool, const int32_t* tables, const 
             h_wide[2 * i] = wide[i].second.first;
             h_wide[2 * i + 1] = wide[i].second.second;
         }
-        p.tables.reserve(nt);
-        p.d_start.reserve(batch);
-        p.d_len.reserve(batch);
-        p.d_row_off.reserve(batch);
-        p.slots.reserve(total);
-        p.row_pos.reserve(total);
-        p.work.reserve(n_work);
-        p.work_wide.reserve(n_wide);
-        st.copy(p.tables.ptr, h_tables, nt, s);
-        st.copy(p.d_start.ptr, h_start, batch, s);
-        st.copy(p.d_len.ptr, h_len, batch, s);
-        st.copy(p.d_row_off.ptr, h_off, batch, s);
-        st.copy(p.slots.ptr, h_slots, total, s);
-        st.copy(p.row_pos.ptr, h_row_pos, total, s);
-        st.copy(p.work.ptr, h_work, n_work, s);
-        st.copy(p.work_wide.ptr, h_wide, n_wide, s);
+        // the device arrays lie as they are staged, so one copy fills them all
+        p.words.reserve(need);
+        p.tables.ptr = p.words.ptr;
+        p.d_start.ptr = p.words.ptr + (h_start - h);
+        p.d_len.ptr = p.words.ptr + (h_len - h);
+        p.d_row_off.ptr = p.words.ptr + (h_off - h);
+        p.slots.ptr = p.words.ptr + (h_slots - h);
+        p.row_pos.ptr = p.words.ptr + (h_row_pos - h);
+        p.work.ptr = p.words.ptr + (h_work - h);
+        p.work_wide.ptr = p.words.ptr + (h_wide - h);
+        st.copy(p.words.ptr, h, need, s);
         st.finish(s);
         p.start_pos.assign(start_pos, start_pos + batch);
         p.num_tokens.assign(num_tokens, num_tokens + batch);

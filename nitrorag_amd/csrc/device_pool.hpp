@@ -60,6 +60,15 @@ struct DeviceBuffer {
     }
 };
 
+// n words from pinned host memory, read by the kernel over the host link
+// (kv_append.hip).
+hipError_t launch_upload_words(int32_t* dst, const int32_t* pinned, size_t n, hipStream_t stream);
+
+// A part of a DeviceBuffer that holds several arrays of one upload.
+struct DeviceWords {
+    int32_t* ptr = nullptr;
+};
+
 // Pinned host staging for uploads: reused once the copies that read it have
 // completed (tracked with an event), so callers may free their arrays at once.
 struct Staging {
@@ -91,7 +100,15 @@ struct Staging {
         }
         return host;
     }
+    // Uploads of up to 256 KB (a batch's tables, positions and work lists) go by
+    // a kernel that reads the staging memory: in the stream it costs a launch,
+    // where a copy waits for another engine on both sides (a decode batch's
+    // three copies: 25 us of GPU time between a pass's kernels).
     void copy(int32_t* dst, const int32_t* src, size_t n, hipStream_t s) {
+        if (n <= 65536) {
+            hip_check(launch_upload_words(dst, src, n, s), "upload launch");
+            return;
+        }
         hip_check(hipMemcpyAsync(dst, src, n * sizeof(int32_t), hipMemcpyHostToDevice, s),
                   "hipMemcpyAsync");
     }
@@ -116,8 +133,15 @@ struct DecodeBatch {
     std::vector<uint32_t> page_mark, page_multi;  // per pool page: upload stamps (shared-page scan)
     uint32_t stamp = 0;
     uint64_t generation = 0;         // bumped by every new batch (work-list cache key)
-    DeviceBuffer<int32_t> tables, pos;
-    DeviceBuffer<int32_t> slots;     // per row: page * 16 + position % 16 (where its K/V row goes)
+    DeviceBuffer<int32_t> words;     // tables, pos and slots, one upload
+    DeviceWords tables, pos;
+    DeviceWords slots;               // per row: page * 16 + position % 16 (where its K/V row goes)
+    void reserve(size_t table_words, size_t rows) {
+        words.reserve(table_words + 2 * rows);
+        tables.ptr = words.ptr;
+        pos.ptr = tables.ptr + table_words;
+        slots.ptr = pos.ptr + rows;
+    }
     // The decode work list last built for this batch, and what it was built for
     // (work_items = 0: longer than the kernel arguments hold).
     DecodeArgItems arg_list;
@@ -144,13 +168,14 @@ struct DecodeBatch {
 struct PrefillBatch {
     int32_t batch = 0, max_pages = 0, total_rows = 0, max_tokens = 0;
     std::vector<int32_t> start_pos, num_tokens, row_off;
-    DeviceBuffer<int32_t> tables, d_start, d_len, d_row_off;
-    DeviceBuffer<int32_t> slots;      // per packed row: page*16 + row-in-page
-    DeviceBuffer<int32_t> row_pos;    // per packed row: its position in the sequence
-    DeviceBuffer<int32_t> work;       // per work item: (seq, first query) pairs
+    DeviceBuffer<int32_t> words;      // the arrays below, one upload
+    DeviceWords tables, d_start, d_len, d_row_off;
+    DeviceWords slots;                // per packed row: page*16 + row-in-page
+    DeviceWords row_pos;              // per packed row: its position in the sequence
+    DeviceWords work;                 // per work item: (seq, first query) pairs
     int32_t work_items = 0;
     int32_t work_block_m = 0;         // query rows per work item the list was built for
-    DeviceBuffer<int32_t> work_wide;  // the same for items of PREFILL_WIDE_ROWS rows
+    DeviceWords work_wide;            // the same for items of PREFILL_WIDE_ROWS rows
     int32_t work_items_wide = 0;
     int32_t max_pos = 0;              // largest position of any row
     // No table entry but a chunk row's own names the page that row lands on:

@@ -164,4 +164,25 @@ hipError_t launch_kv_scatter_rows(float* k_pool, float* v_pool, const float* k, 
     return hipGetLastError();
 }
 
+namespace {
+// 16 bytes per thread, the last few words one each; grid-stride not needed (the
+// caller's n is bounded by the upload limit).
+__global__ __launch_bounds__(256) void upload_words_kernel(int32_t* __restrict__ dst, const int32_t* __restrict__ src,
+                                                           int n) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n / 4)
+        reinterpret_cast<int4*>(dst)[i] = reinterpret_cast<const int4*>(src)[i];
+    else if (i - n / 4 < n % 4)
+        dst[n / 4 * 4 + i - n / 4] = src[n / 4 * 4 + i - n / 4];
+}
+}  // namespace
+
+hipError_t launch_upload_words(int32_t* dst, const int32_t* pinned, size_t n, hipStream_t stream) {
+    if (n == 0) return hipSuccess;
+    if (n > (1u << 30) || ((uintptr_t)dst | (uintptr_t)pinned) % 16) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(upload_words_kernel, dim3((unsigned)((n / 4 + 3 + 255) / 256)), dim3(256), 0, stream, dst, pinned,
+                       (int)n);
+    return hipGetLastError();
+}
+
 }  // namespace nitro
