@@ -628,7 +628,7 @@ __global__ __launch_bounds__(64 * QT * KSPLIT) void paged_attn_prefill_mfma_kern
 // at position 0), every key new.  APPEND 2: chunks after cached keys; a key
 // below its chunk's start is read from the pool, the others from the new
 // rows, chosen per key (a tile may hold both).
-template <int HDL, int HD, bool FULL, int VP, int QT, int KSPLIT, int BNM, int APPEND>
+template <int HDL, int HD, bool FULL, int VP, int QT, int KSPLIT, int BNM, int APPEND, bool DB>
 // Up to hd 64 two workgroups share a CU (LDS), which takes at most 128
 // VGPRs (4 waves per SIMD); larger heads run one workgroup per CU.
 __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn_prefill_x3_kernel(PrefillLaunch a) {
@@ -654,9 +654,10 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
     constexpr int KPLANE = BNM * KST, VPLANE = HD * VST;
     static_assert((KSPLIT - 1) * QT * 16 * HD * 4 <= (3 * KPLANE + VP * VPLANE) * 2, "partials fit the tile planes");
     // K in three bf16 planes, V^T in VP
-    __shared__ __attribute__((aligned(16))) uint16_t kv_lds[3 * KPLANE + VP * VPLANE];
-    uint16_t* const k_lds = kv_lds;
-    uint16_t* const v_lds = kv_lds + 3 * KPLANE;
+    // DB: two buffers, so that a tile is staged while the one before is computed.
+    static_assert(!DB || KSPLIT == 1, "the partials of several key groups take the place of one buffer");
+    constexpr int BUF = 3 * KPLANE + VP * VPLANE;
+    __shared__ __attribute__((aligned(16))) uint16_t kv_lds[(DB ? 2 : 1) * BUF];
     __shared__ int32_t s_table[TABLE_LDS];
     __shared__ float s_ml[KSPLIT > 1 ? QT * (KSPLIT - 1) * 16 * 2 : 1];
     __shared__ int32_t s_wave_bad[NT / 64];
@@ -929,117 +930,42 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
                             w.x * a.qscale, w.y * a.qscale, w.z * a.qscale, w.w * a.qscale};
         split3(v, qp[0][c], qp[1][c], qp[2][c]);
     }
-    for (int tile = 0; tile < n_tiles; tile++) {
-        __syncthreads();  // previous tile fully consumed
-        // Staging and the next tile's loads at a raised wave priority: of the
-        // waves sharing a SIMD (two workgroups), the ones staging a tile issue
-        // before the ones computing, so the tile's barrier is reached and the
-        // next loads go out sooner (8 prompts of 128-1024 tokens at 12 x 64:
-        // 50.3 vs 51.6-52.5 us by trace; priority 3, or priority 1 also around
-        // the matrix-core blocks, were no better).
-        __builtin_amdgcn_s_setprio(1);
-        // four values as two bf16 planes (hi, mid), one 8-byte store each
-        auto stage4v = [](uint16_t* dst, int plane, const float (&v)[4]) {
-            const float r0 = v[0] - upper16(v[0]), r1 = v[1] - upper16(v[1]);
-            const float r2 = v[2] - upper16(v[2]), r3 = v[3] - upper16(v[3]);
-            *reinterpret_cast<uint2*>(dst) = make_uint2(bf16_pair(v[0], v[1]), bf16_pair(v[2], v[3]));
-            *reinterpret_cast<uint2*>(dst + plane) = make_uint2(bf16_pair(r0, r1), bf16_pair(r2, r3));
-        };
-        // four values as three bf16 planes, one 8-byte store each
-        auto stage4 = [](uint16_t* dst, int plane, const float (&v)[4]) {
-            const float r0 = v[0] - upper16(v[0]), r1 = v[1] - upper16(v[1]);
-            const float r2 = v[2] - upper16(v[2]), r3 = v[3] - upper16(v[3]);
-            const float l0 = r0 - upper16(r0), l1 = r1 - upper16(r1);
-            const float l2 = r2 - upper16(r2), l3 = r3 - upper16(r3);
-            *reinterpret_cast<uint2*>(dst) = make_uint2(bf16_pair(v[0], v[1]), bf16_pair(v[2], v[3]));
-            *reinterpret_cast<uint2*>(dst + plane) = make_uint2(bf16_pair(r0, r1), bf16_pair(r2, r3));
-            *reinterpret_cast<uint2*>(dst + 2 * plane) = make_uint2(bf16_pair(l0, l1), bf16_pair(l2, l3));
-        };
-        // the masks are applied only where a wave holds a row to zero
-        // (the last tile of a sequence, bad pages): other tiles skip the selects
-        auto stage_tile = [&](bool masked) {
-#pragma unroll
-            for (int i = 0; i < LOADS; i++) {
-                const int f = threadIdx.x + i * NT;
-                const int r = f / F4, col = f % F4;
-                const bool ok = !masked || ((kmask >> i) & 1);
-                const float kv4[4] = {ok ? kreg[i].x : 0.f, ok ? kreg[i].y : 0.f, ok ? kreg[i].z : 0.f,
-                                      ok ? kreg[i].w : 0.f};
-                if (HDL == HD || col * 4 < HD) stage4(&k_lds[r * KST + col * 4], KPLANE, kv4);
-            }
-#pragma unroll
-            for (int i = 0; i < VSLOTS; i++) {
-                const int sl = threadIdx.x + i * NT;
-                float v4[4];
-#pragma unroll
-                for (int e = 0; e < 4; e++) v4[e] = !masked || ((vmask >> (4 * i + e)) & 1) ? vreg[i][e] : 0.f;
-                if (HDL == HD || vslot < HD) {
-                    uint16_t* dst = &v_lds[vslot * VST + 4 * (sl / HDL)];
-                    if constexpr (VP == 3)
-                        stage4(dst, VPLANE, v4);
-                    else
-                        stage4v(dst, VPLANE, v4);
-                }
-            }
-        };
-        if constexpr (APPEND == 1) {
-            if (any_bad) {  // block-uniform: keys on pages outside the pool are staged as zero
-#pragma unroll
-                for (int i = 0; i < LOADS; i++) {
-                    const int key = tile * BNM + (int)(threadIdx.x + i * NT) / F4;
-                    if (s_table[min(key, last_pos) >> 4] < 0) kmask &= ~(1u << i);
-                }
-#pragma unroll
-                for (int i = 0; i < VSLOTS; i++) {
-                    const int key0 = tile * BNM + 4 * ((int)(threadIdx.x + i * NT) / HDL);  // 4 keys, one page
-                    if (s_table[min(key0, last_pos) >> 4] < 0) vmask &= ~(0xFu << (4 * i));
-                }
-            }
+    // DB: one of the two buffers.
+    auto stage = [&](const int& tile) __attribute__((always_inline)) {
+        uint16_t* const k_lds = kv_lds + (tile & 1) * BUF;
+        uint16_t* const v_lds = k_lds + 3 * KPLANE;
+#include "prefill_stage_tile.inc"
+    };
+    // DB: iteration t stages tile t + 1, the first half of the waves (one per
+    // SIMD) before they compute tile t, the others after: a SIMD's two waves then
+    // alternate between the matrix cores and the staging's VALU work.
+    const bool early = DB && wave < NT / 128;
+    auto stage_next = [&](auto tile) __attribute__((always_inline)) {  // (generic: only DB has it)
+        if (tile + 1 < n_tiles) {
+            stage(tile + 1);
+            if (tile + 2 < n_tiles) fetch(tile + 2);
+            __builtin_amdgcn_s_setprio(0);
         }
-        if (__builtin_amdgcn_ballot_w64(kmask != KFULL || vmask != VFULL) != 0)  // wave-uniform
-            stage_tile(true);
-        else
-            stage_tile(false);
-        if constexpr (APPEND) {
-            // The append, by the workgroup of the first head of each kv group:
-            // the tile's keys that are this item's query rows (positions
-            // own_first .. last_pos) are stored from the registers they were
-            // just loaded into, at the pool address the pool form reads them
-            // from, as streaming stores (nothing in the launch reads them; 0.6
-            // us of 57 on 8 prompts of 128-1024 tokens at 12 x 64).  A row on a
-            // page outside the pool is counted once (kv head 0, its first
-            // column) and skipped, as the scatter does.
-            if (appends && tile * BNM + BNM > own_first) {  // block-uniform
-                char* const kw = const_cast<char*>(kb);
-                char* const vw = const_cast<char*>(vb);
-#pragma unroll
-                for (int i = 0; i < LOADS; i++) {
-                    const int f = threadIdx.x + i * NT;
-                    const int key = tile * BNM + f / F4;
-                    if (kcol_ok && key >= own_first && key <= last_pos) {
-                        const int page = s_table[key >> 4];
-                        if (page >= 0)
-                            __builtin_nontemporal_store(f32x4{kreg[i].x, kreg[i].y, kreg[i].z, kreg[i].w},
-                                                        reinterpret_cast<f32x4*>(kw + (size_t)(uint32_t)page * stride_b));
-                        else if (kv_h == 0 && kslot == 0)
-                            atomicAdd(a.bad_pages, 1);
-                    }
-                }
-#pragma unroll
-                for (int i = 0; i < VSLOTS; i++) {
-                    const int key0 = tile * BNM + 4 * ((int)(threadIdx.x + i * NT) / HDL);  // 4 keys, one page
-                    const int page = s_table[min(key0, last_pos) >> 4];
-#pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        if (vcol_ok && key0 + e >= own_first && key0 + e <= last_pos && page >= 0)
-                            __builtin_nontemporal_store(
-                                vreg[i][e], reinterpret_cast<float*>(vw + (size_t)(uint32_t)page * stride_b + e * vrow_b));
-                }
-            }
-        }
-        __syncthreads();
-        if (tile + 1 < n_tiles) fetch(tile + 1);
+    };
+    if constexpr (DB) {
+        stage(0);
+        if (n_tiles > 1) fetch(1);
         __builtin_amdgcn_s_setprio(0);
+    }
+    for (int tile = 0; tile < n_tiles; tile++) {
+        __syncthreads();  // the tile before is consumed (DB: and this one staged)
+        if constexpr (DB) {
+            if (early) stage_next(tile);
+        } else {
+            uint16_t* const k_lds = kv_lds;
+            uint16_t* const v_lds = kv_lds + 3 * KPLANE;
+#include "prefill_stage_tile.inc"
+            __syncthreads();
+            if (tile + 1 < n_tiles) fetch(tile + 1);
+            __builtin_amdgcn_s_setprio(0);
+        }
+        uint16_t* const k_lds = kv_lds + (DB ? (tile & 1) * BUF : 0);
+        uint16_t* const v_lds = k_lds + 3 * KPLANE;
 
         int nvb = 0;
 #pragma unroll
@@ -1158,6 +1084,8 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
                 }
             }
         }
+        if constexpr (DB)
+            if (!early) stage_next(tile);
     }
 
     lsum = sum_over_rows(lsum);
@@ -1207,17 +1135,35 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
 }
 
 // One instance of the bf16 matrix-core kernel; APPENDS: its appending forms are built.
-template <int HDL, int HD, bool FULL, int VP, int QT, int KSPLIT, int BNM, bool APPENDS>
-void launch_x3(const PrefillLaunch& a, dim3 grid, hipStream_t stream) {
+template <int HDL, int HD, bool FULL, int VP, int QT, int KSPLIT, int BNM, bool APPENDS, bool DB>
+void launch_x3_as(const PrefillLaunch& a, dim3 grid, hipStream_t stream) {
     const dim3 block(64 * QT * KSPLIT);
     if constexpr (APPENDS) {
         if (a.k_new && a.append_mixed)
-            hipLaunchKernelGGL((paged_attn_prefill_x3_kernel<HDL, HD, FULL, VP, QT, KSPLIT, BNM, 2>), grid, block, 0, stream, a);
+            hipLaunchKernelGGL((paged_attn_prefill_x3_kernel<HDL, HD, FULL, VP, QT, KSPLIT, BNM, 2, DB>), grid, block, 0, stream, a);
         else if (a.k_new)
-            hipLaunchKernelGGL((paged_attn_prefill_x3_kernel<HDL, HD, FULL, VP, QT, KSPLIT, BNM, 1>), grid, block, 0, stream, a);
+            hipLaunchKernelGGL((paged_attn_prefill_x3_kernel<HDL, HD, FULL, VP, QT, KSPLIT, BNM, 1, DB>), grid, block, 0, stream, a);
         if (a.k_new) return;
     }
-    hipLaunchKernelGGL((paged_attn_prefill_x3_kernel<HDL, HD, FULL, VP, QT, KSPLIT, BNM, 0>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((paged_attn_prefill_x3_kernel<HDL, HD, FULL, VP, QT, KSPLIT, BNM, 0, DB>), grid, block, 0, stream, a);
+}
+
+// Two K/V buffers where a workgroup has its CU to itself anyway (heads of 65..128)
+// and the batch reaches DB_MIN_POS: 4000 tokens at 32/8 x 128 653 -> 599 us per
+// layer, chunks of 384-512 after up to 4096 cached tokens 289 -> 280, 300 tokens
+// at 8 x 128 32 -> 29, 4000 at 32 x 80 658 -> 623.  In short loops the first
+// staged tile waits for loads that have only just gone out: 16 chunks of 64-128
+// tokens took 41.2 -> 45.0 us at 32 x 80, 36.9 -> 37.5 at 32/8 x 128.
+constexpr int DB_MIN_POS = 256;
+template <int HDL, int HD, bool FULL, int VP, int QT, int KSPLIT, int BNM, bool APPENDS>
+void launch_x3(const PrefillLaunch& a, dim3 grid, hipStream_t stream) {
+    if constexpr (KSPLIT == 1 && HD <= 128) {
+        if (a.max_pos >= DB_MIN_POS) {
+            launch_x3_as<HDL, HD, FULL, VP, QT, KSPLIT, BNM, APPENDS, true>(a, grid, stream);
+            return;
+        }
+    }
+    launch_x3_as<HDL, HD, FULL, VP, QT, KSPLIT, BNM, APPENDS, false>(a, grid, stream);
 }
 
 }  // namespace
