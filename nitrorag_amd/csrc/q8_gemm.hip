@@ -304,6 +304,17 @@ __global__ __launch_bounds__(64 * GEMM_WAVES, GEMM_NT == 8 ? 2 : 3) void q8_gemm
             for (int t = 0; t < GEMM_NT; t++) acc[m][t] += sums[wave][m * GEMM_NT + t][lane];
     }
 
+    // The next norm's weights of the lane's split columns, loaded before any store.
+    float out_w[EPI == Q8Epilogue::Residual ? GEMM_BN / 32 : 1][8];
+    if constexpr (EPI == Q8Epilogue::Residual) {
+        if (out.planes && out.weight) {  // uniform
+#pragma unroll
+            for (int j = 0; j < GEMM_BN / 32; j++)
+#pragma unroll
+                for (int i = 0; i < 8; i++) out_w[j][i] = out.weight[min(row0 + 32 * j + 8 * lg, d - 8) + i];
+        }
+    }
+
     // Lane l holds out[b0 + 16m + 4*(l/16) + i][16t + l%16] in acc[m][t][i].
 #pragma unroll
     for (int m = 0; m < GEMM_MT; m++) {
@@ -330,7 +341,7 @@ __global__ __launch_bounds__(64 * GEMM_WAVES, GEMM_NT == 8 ? 2 : 3) void q8_gemm
                 const float* src = rows + lr * (COLS + 4) + 32 * j + 8 * lg;
                 float v[8];
 #pragma unroll
-                for (int i = 0; i < 8; i++) v[i] = out.weight ? src[i] * out.weight[k + i] : src[i];
+                for (int i = 0; i < 8; i++) v[i] = EPI == Q8Epilogue::Residual && out.weight ? src[i] * out_w[j][i] : src[i];
                 bf16x8 p[3];
                 split3(v, p[0], p[1], p[2]);
                 char* dst = out.planes + split_at(b0 + 16 * m + lr, k, out.nb);
@@ -354,15 +365,20 @@ __global__ __launch_bounds__(64 * GEMM_WAVES, GEMM_NT == 8 ? 2 : 3) void q8_gemm
         } else if constexpr (EPI == Q8Epilogue::Residual) {
             // x += product; the squares of the new entries are added over each
             // 16-row tile's 16 lanes (one partial per batch row and tile)
+            // (every x is loaded before the first store: a load behind a store
+            // that may alias it waits its turn, one round trip per tile)
+            float xv[GEMM_NT][4];
+#pragma unroll
+            for (int t = 0; t < GEMM_NT; t++)
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    xv[t][i] = grp.out[0][(size_t)min(bm + i, batch - 1) * d + min(row0 + 16 * t + lr, d - 1)];
 #pragma unroll
             for (int t = 0; t < GEMM_NT; t++) {
                 const int row = row0 + 16 * t + lr;
-                float xv[4];
-#pragma unroll
-                for (int i = 0; i < 4; i++) xv[i] = grp.out[0][(size_t)min(bm + i, batch - 1) * d + min(row, d - 1)];
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    const float v = xv[i] + acc[m][t][i];
+                    const float v = xv[t][i] + acc[m][t][i];
                     const bool ok = bm + i < batch && row < d;
                     if (ok) grp.out[0][(size_t)(bm + i) * d + row] = v;
                     rows[(4 * lg + i) * (COLS + 4) + 16 * t + lr] = v;
@@ -374,27 +390,38 @@ __global__ __launch_bounds__(64 * GEMM_WAVES, GEMM_NT == 8 ? 2 : 3) void q8_gemm
             }
             if (out.planes) write_split();  // uniform
         } else if constexpr (EPI == Q8Epilogue::Rope) {
-            // RoPE pairs are adjacent weight rows, so adjacent lanes
+            // RoPE pairs are adjacent weight rows, so adjacent lanes; the rows'
+            // slots and angles are loaded before the first store, as above
+            RopeRow rr[4];
+            float cs[4][GEMM_NT], sn[4][GEMM_NT];
+#pragma unroll
+            for (int i = 0; i < 4; i++) rr[i] = rope_row(rope, min(bm + i, batch - 1));
+            if (member < 2) {  // uniform
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+#pragma unroll
+                    for (int t = 0; t < GEMM_NT; t++) {
+                        const size_t f = (size_t)rr[i].pos * (rope.head_dim >> 1) + ((row0 + 16 * t + lr) % rope.head_dim >> 1);
+                        cs[i][t] = rope.freq_real[f];
+                        sn[i][t] = rope.freq_imag[f];
+                    }
+            }
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int b = bm + i;
-                const RopeRow rr = rope_row(rope, min(b, batch - 1));
 #pragma unroll
                 for (int t = 0; t < GEMM_NT; t++) {
                     const int row = row0 + 16 * t + lr;
                     const float mine = acc[m][t][i], other = __shfl_xor(mine, 1);
                     if (b >= batch || row >= d) continue;
                     float v = mine;
-                    if (member < 2) {
-                        const bool odd = row & 1;
-                        const float2 q = rotate_pair(rope, rr.pos, row & ~1, odd ? other : mine, odd ? mine : other);
-                        v = odd ? q.y : q.x;
-                    }
+                    if (member < 2)  // rotate_pair's (x*c - y*sn, x*sn + y*c)
+                        v = row & 1 ? other * sn[i][t] + mine * cs[i][t] : mine * cs[i][t] - other * sn[i][t];
                     if (member == 0) {
                         grp.out[0][(size_t)b * d + row] = v;
-                    } else if (rr.page_ok) {
+                    } else if (rr[i].page_ok) {
                         float* pool = member == 1 ? rope.k_pool : rope.v_pool;
-                        pool[(size_t)rr.page * rope.page_stride + rope.layer_off + (size_t)rr.in_page * d + row] = v;
+                        pool[(size_t)rr[i].page * rope.page_stride + rope.layer_off + (size_t)rr[i].in_page * d + row] = v;
                     } else if (member == 1 && row == 0) {
                         atomicAdd(rope.bad_pages, 1);  // once per row
                     }
