@@ -236,7 +236,7 @@ int nitro_kv_append_prefill(nitro_kvpool* pool, int32_t layer, const float* k, c
 /* Causal paged prefill attention — src/model_q8.cpp:485-523.  q, out: device
  * [total_tokens][n_heads*head_dim]; the token at pos attends keys 0..pos
  * (prefix-hit pages, earlier chunks and this chunk's own rows).  head_dim: any
- * multiple of 4 from 4 to 256 (32, 64 and 128 run on the matrix cores). */
+ * multiple of 4 from 4 to 256. */
 int nitro_paged_attn_prefill(nitro_kvpool* pool, int32_t layer, const float* q, float* out,
                              int32_t n_heads, int32_t n_kv_heads, int32_t head_dim, void* stream);
 
@@ -244,7 +244,7 @@ int nitro_paged_attn_prefill(nitro_kvpool* pool, int32_t layer, const float* q, 
  * reference's prefill layer step, src/model_q8.cpp:473-484 then :485-523
  * (nitro_kv_append_prefill followed by nitro_paged_attn_prefill, with the same
  * pool contents and output).  k, v: device [total_tokens][kv_dim].  With the
- * matrix-core kernel (head_dim 32, 64, 128), positions below 32768, and no
+ * bf16 matrix-core kernel (head_dim 32, 64, 68..96, 128), positions below 32768, and no
  * page that a chunk row lands on named by any other table entry (checked at
  * upload), one launch reads each chunk's keys from k / v (keys cached before
  * start_pos from the pool) and appends the chunk: fresh prompts, later chunks

@@ -607,9 +607,9 @@ __global__ __launch_bounds__(64 * QT * KSPLIT) void paged_attn_prefill_mfma_kern
 // thread's column is the same in every load.  Columns between the head size
 // and HD are staged as zero.  These sizes ran on the VALU kernel before, which
 // is bound by its FMAs and LDS reads: 6 prompts of 50-700 tokens at 16 x 96
-// 445 -> 70 us per layer with the append, 16 x 256 900 -> 160, 32 x 80 450 ->
-// 125, 12 x 48 135 -> 50; one 4000-token prompt at 16 x 96 2.43 -> 0.33 ms;
-// one token the same.
+// 445 -> 56 us per layer with the append, 16 x 256 905 -> 147, 32 x 80 460 ->
+// 113, 12 x 48 138 -> 54; one 4000-token prompt at 16 x 96 2.43 -> 0.32 ms;
+// one token no slower.
 // A workgroup serves one work item of 16*QT query rows (QT = 8: 128 rows,
 // the wide work list, so each staged tile serves twice the queries) with QT
 // query sub-tiles x KSPLIT key groups of waves.

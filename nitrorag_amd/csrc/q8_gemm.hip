@@ -38,11 +38,11 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 //    (2-norm) at n = 768 / 2048 / 4096 / 11008, as q8_mma_kernel's 0.80 / 0.97
 //    / 1.2 / 1.74, which adds eight waves' chains; one chain gave 1.0e-7 at 768.
 // Bound by the matrix cores and, at n = 768, by the first and last blocks of a
-// tile: w1/w3 of 5520 rows at 768 x 2048 370 -> 112 us (0.93 PFLOP/s of bf16
-// products, three per multiply), wq/wk/wv 216 -> 84, wo 99 -> 39; 1600 rows at
-// 4096 x 11008 are at 46% of the matrix cores' cycles (a plain 8192^3 bf16
-// product reaches 50%).  Prompts of 8 users, 110M-parameter shapes: 11.96 ->
-// 5.0 ms; q8_matmul of 1024 rows, 4096 x 11008, three products: 5.18 -> 1.70 ms.
+// tile: w1/w3 of 5520 rows at 768 x 2048 370 -> 117 us with hb written split
+// (0.89 PFLOP/s of bf16 products, three per multiply), wq/wk/wv 216 -> 89, wo
+// 99 -> 40; 1600 rows at 4096 x 11008 are at 46% of the matrix cores' cycles (a
+// plain 8192^3 bf16 product reaches 50%).  Prompts of 8 users, 110M-parameter
+// shapes: 11.96 -> 4.8 ms; q8_matmul of 1024 rows, 4096 x 11008, three products: 5.18 -> 1.70 ms.
 constexpr int GEMM_WAVES = 4;
 constexpr int GEMM_BM = 32 * GEMM_WAVES;
 constexpr int GEMM_MT = 2;            // 16-row batch tiles per wave
