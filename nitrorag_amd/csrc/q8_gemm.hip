@@ -42,7 +42,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // (0.89 PFLOP/s of bf16 products, three per multiply), wq/wk/wv 216 -> 89, wo
 // 99 -> 40; 1600 rows at 4096 x 11008 are at 46% of the matrix cores' cycles (a
 // plain 8192^3 bf16 product reaches 50%).  Prompts of 8 users, 110M-parameter
-// shapes: 11.96 -> 4.8 ms; q8_matmul of 1024 rows, 4096 x 11008, three products: 5.18 -> 1.70 ms.
+// shapes: 11.96 -> 4.6 ms; q8_matmul of 1024 rows, 4096 x 11008, three products: 5.18 -> 1.10 ms.
 constexpr int GEMM_WAVES = 4;
 constexpr int GEMM_BM = 32 * GEMM_WAVES;
 constexpr int GEMM_MT = 2;            // 16-row batch tiles per wave
@@ -108,11 +108,19 @@ __global__ __launch_bounds__(64 * GEMM_WAVES, GEMM_NT == 8 ? 2 : 3) void q8_gemm
                         : row * nb * Q8_BLOCK_BYTES + 4 + 8 * c;
         wdst[u] = w_at(r, c);
     }
-    uint32_t soff[GEMM_NT];  // the scale of this lane's row of each tile
+    // A block's scales, one per lane of each 64 weight rows: a tile's are handed
+    // to its lanes by a permute.  (Loaded per tile, 16 rows by each of 4 lane
+    // groups, they took twice the address slots of row-major x: three products of
+    // 1024 rows at 4096 x 11008 1.70 -> 1.10 ms, 8 prompts of the 110M-parameter
+    // shapes 4.72 -> 4.56 ms.)
+    constexpr int SC = GEMM_NT / 4;
+    const uint8_t* sbase[SC];
 #pragma unroll
-    for (int t = 0; t < GEMM_NT; t++) {
-        const uint32_t row = wrow_of(16 * t + lr);
-        soff[t] = TILED ? row / 16 * nb * Q8_TILE_BYTES + 4 * (row % 16) : row * nb * Q8_BLOCK_BYTES;
+    for (int u = 0; u < SC; u++) {
+        const int rr = 64 * u + lane;
+        const uint32_t row = wrow_of(rr);
+        sbase[u] = base_of(SWIGLU ? rr / MROWS : member) +
+                   (TILED ? row / 16 * nb * Q8_TILE_BYTES + 4 * (row % 16) : row * nb * Q8_BLOCK_BYTES);
     }
     // x of the wave's two 16-row tiles: their planes (PRE; tiles clamped), or the
     // batch rows this lane feeds (clamped: never stored).
@@ -138,7 +146,7 @@ __global__ __launch_bounds__(64 * GEMM_WAVES, GEMM_NT == 8 ? 2 : 3) void q8_gemm
     };
     struct XRound {
         u32x4 v[GEMM_MT][PRE ? 3 : 2];  // PRE: hi, mid, lo; else 8 floats
-        float sc[GEMM_NT];
+        float sc[SC];
     };
     auto load_w = [&](WRound& R, int blk) __attribute__((always_inline)) {
         const size_t step = (size_t)((uint32_t)walk(blk) * BSTEP);
@@ -163,8 +171,7 @@ __global__ __launch_bounds__(64 * GEMM_WAVES, GEMM_NT == 8 ? 2 : 3) void q8_gemm
             for (int i = 0; i < (PRE ? 3 : 2); i++)
                 R.v[m][i] = *reinterpret_cast<const u32x4*>(xb + xoff[m] + (PRE ? 1024 : 16) * i);
 #pragma unroll
-        for (int t = 0; t < GEMM_NT; t++)
-            R.sc[t] = *reinterpret_cast<const float*>(base_of(SWIGLU ? t / (GEMM_NT / 2) : member) + (size_t)((uint32_t)blk * BSTEP) + soff[t]);
+        for (int u = 0; u < SC; u++) R.sc[u] = *reinterpret_cast<const float*>(sbase[u] + (size_t)((uint32_t)blk * BSTEP));
     };
     auto stage_w = [&](const WRound& R, int buf) __attribute__((always_inline)) {
 #pragma unroll
@@ -239,8 +246,10 @@ __global__ __launch_bounds__(64 * GEMM_WAVES, GEMM_NT == 8 ? 2 : 3) void q8_gemm
                     for (int i = 0; i < 4; i++) acc[m][tl + u][i] = fmaf(late_sc[u], late[m][u][i], acc[m][tl + u][i]);
                     late[m][u] = s[m][u];
                 }
-            late_sc[0] = xc.sc[t];
-            late_sc[1] = xc.sc[t + 1];
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+                late_sc[u] = __int_as_float(
+                    __builtin_amdgcn_ds_bpermute(4 * (16 * ((t + u) % 4) + lr), __float_as_int(xc.sc[t / 4])));
             if (t == 0) stage_w(wn, (blk + 1) & 1);
             if (t == 2) load_w(wn, blk + 3);
             if (t + 2 < GEMM_NT) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // LDS reads
@@ -499,8 +508,8 @@ bool launch_q8_gemm(Q8Epilogue epilogue, const Q8Group& grp, const float* x, con
     // however full it is).  wo at 5520 x 768: 264 wide workgroups 51 us, 528
     // narrow 39; at 1600 x 4096, 416 wide ones fit a round and 832 narrow ones
     // do not: 4.20 ms per pass against 4.38.  Where a wave splits x itself, it
-    // does so twice as often with 64 (1024 rows, 4096 x 11008: 2.08 ms against
-    // 1.70), hence the 0.75.
+    // does so twice as often with 64 (1024 rows, 4096 x 11008, with scales still
+    // loaded per tile: 2.08 ms against 1.70), hence the 0.75.
     constexpr int CUS = 256;
     const long long panels = (batch + GEMM_BM - 1) / GEMM_BM;
     const long long wide = panels * columns(128), slim = panels * columns(64);
@@ -510,10 +519,10 @@ bool launch_q8_gemm(Q8Epilogue epilogue, const Q8Group& grp, const float* x, con
     const long long wgs = narrow ? slim : wide;
     // A round takes about 1 us per block (1.3 with 128 rows) at any size, the
     // small-batch kernel rows x outputs x n / 26.5e6 us, so this kernel pays
-    // from about 830,000 outputs per round.  Measured on both sides: three
-    // products of 128 rows at 4096 x 11008 667 us there, 608 with the rule, 952
-    // all here; 256 rows 58 / 57 / 107 at 768 x 2048, 344 / 312 / 477 at 2048 x
-    // 5632, 1325 / 805 / 958 at 4096 x 11008.
+    // from about 830,000 outputs per round.  Three products there and with the
+    // rule: 128 rows at 4096 x 11008 667 / 488 us; 256 rows at 2048 x 5632 344 /
+    // 249, at 4096 x 11008 1325 / 682, at 768 x 2048 58 / 58 (none taken; all of
+    // them taken lost at 768, as 128 rows of w2 at 4096 x 11008 did).
     double outputs = 0;
     for (int m = 0; m < members; m++) outputs += (double)batch * grp.d[m];
     if (wgs > (1ll << 30) || outputs < (narrow ? 830e3 * slim_rounds : 1080e3 * wide_rounds)) return false;
