@@ -1191,6 +1191,15 @@ constexpr int mma_unroll() {
 constexpr int MMA_MAX_BT = 2;       // batch tiles per workgroup (more rows: more workgroups along y)
 constexpr int MMA_NORM_MAX_N = 8192;  // rms weights staged in LDS (larger n: the fp32 kernel)
 
+// Whether q8_mma_kernel's 32-bit byte offsets reach everything it reads: a
+// matrix from its start, x in rows from a workgroup's first row (in split form:
+// from its start).
+bool mma_offsets_fit(size_t d, size_t n, size_t batch, bool split) {
+    constexpr size_t LIMIT = 1ull << 32;
+    return q8_tiled_bytes(d, n) < LIMIT &&
+           (split ? q8_split_bytes(batch, n) < LIMIT : 16 * MMA_MAX_BT * n * sizeof(float) < LIMIT);
+}
+
 // One round of a wave: weights and x of U blocks.
 template <int NMAT, int BT, int U, bool PRE>
 struct MmaRound {
@@ -1218,8 +1227,8 @@ __global__ __launch_bounds__(64 * MMA_WAVES) void q8_mma_kernel(Q8Group grp, con
     // Lanes past the batch read the last batch row and rows past a member's
     // end read its last row (finite values, never stored); blocks past the
     // row read the last block, and compute gives them scale 0.
-    // (32-bit offsets from the uniform bases: the launcher keeps each matrix
-    // and x under 2^32 bytes).  Block blk of this lane: its 8 weights at
+    // (32-bit byte offsets from the uniform bases: mma_offsets_fit).  Block blk
+    // of this lane: its 8 weights at
     // qoff + blk * BSTEP, its row's scale at soff + blk * BSTEP.
     constexpr uint32_t BSTEP = TILED ? 576 : Q8_BLOCK_BYTES;
     const uint8_t* wbase[NMAT];
@@ -1238,10 +1247,11 @@ __global__ __launch_bounds__(64 * MMA_WAVES) void q8_mma_kernel(Q8Group grp, con
             soff[m] = row;
         }
     }
-    // x: byte offset of this lane's run of block 0 (PRE: batch tiles clamped; in a
-    // tile of up to 8 rows, lanes of rows 8..15 reread rows 0..7, so that half
-    // the lines are read)
-    const char* const xb = static_cast<const char*>(xin);
+    // x: byte offset of this lane's run of block 0, in rows from the workgroup's
+    // first one, which the 64-bit base is at (PRE: from the start, batch tiles
+    // clamped; in a tile of up to 8 rows, lanes of rows 8..15 reread rows 0..7, so
+    // that half the lines are read)
+    const char* const xb = static_cast<const char*>(xin) + (PRE ? 0 : (size_t)b0 * n * 4);
     uint32_t xoff[BT];
 #pragma unroll
     for (int t = 0; t < BT; t++)
@@ -1249,7 +1259,7 @@ __global__ __launch_bounds__(64 * MMA_WAVES) void q8_mma_kernel(Q8Group grp, con
             xoff[t] = (uint32_t)min(b0 / 16 + t, (batch - 1) / 16) * nb * Q8_SPLIT_BYTES +
                       16 * (batch - (b0 + t * 16) <= 8 ? lane & ~8 : lane);
         else
-            xoff[t] = ((uint32_t)min(b0 + t * 16 + r, batch - 1) * n + 8 * g) * 4;
+            xoff[t] = ((uint32_t)(min(b0 + t * 16 + r, batch - 1) - b0) * n + 8 * g) * 4;
     constexpr uint32_t XSTEP = PRE ? Q8_SPLIT_BYTES : Q8_BLOCK * 4;
     f32x4 acc[NMAT][BT];
 #pragma unroll
@@ -1598,8 +1608,7 @@ void launch_group(const Q8Group& grp, const float* x, int batch, int n, int dmax
     }
     constexpr Q8Epilogue EPI = ROPE ? Q8Epilogue::Rope : RESID ? Q8Epilogue::Residual : SWIGLU ? Q8Epilogue::SwiGlu : Q8Epilogue::Store;
     if (use_mma() && launch_q8_gemm(EPI, grp, x, split, batch, n, nm, rs, rp, stream)) return;
-    // the bf16 kernel addresses weights and x with 32-bit offsets
-    const bool mma_fits = q8_tiled_bytes(dmax, n) < (1ull << 32) && (size_t)batch * n < (1ull << 32) &&
+    const bool mma_fits = mma_offsets_fit(dmax, n, batch, split.in != nullptr) && (size_t)batch * n < (1ull << 32) &&
                           (!NORM || split.in || n <= MMA_NORM_MAX_N);
     if (use_mma() && mma_fits) {
         bool tiled = true;
