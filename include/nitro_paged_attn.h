@@ -236,7 +236,9 @@ int nitro_kv_append_prefill(nitro_kvpool* pool, int32_t layer, const float* k, c
 /* Causal paged prefill attention — src/model_q8.cpp:485-523.  q, out: device
  * [total_tokens][n_heads*head_dim]; the token at pos attends keys 0..pos
  * (prefix-hit pages, earlier chunks and this chunk's own rows).  head_dim: any
- * multiple of 4 from 4 to 256. */
+ * multiple of 4 from 4 to 256.  Infinite q, k and v entries are taken as fp32
+ * arithmetic has them, except at head_dim 32, 64 and 128: there each one makes
+ * the outputs that it meets NaN. */
 int nitro_paged_attn_prefill(nitro_kvpool* pool, int32_t layer, const float* q, float* out,
                              int32_t n_heads, int32_t n_kv_heads, int32_t head_dim, void* stream);
 

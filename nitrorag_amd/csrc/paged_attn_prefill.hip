@@ -573,6 +573,83 @@ __global__ __launch_bounds__(64 * QT * KSPLIT) void paged_attn_prefill_mfma_kern
     }
 }
 
+// Row `at` of this workgroup's work item by one wave in fp32 VALU sums, keys a lane
+// each for the scores and output columns a lane each.  For the rows that the bf16
+// splits leave NaN: the parts of an infinity are infinity and NaN, so an infinite
+// Q, K or V entry makes every output that it meets NaN there, where in fp32 a
+// score of minus infinity has weight 0 and an infinite V an infinite output, and
+// keys past the row's position do not reach it at all.  (A NaN input gives NaN
+// again.)  Finite inputs whose scores do not overflow never come here; finding out
+// costs them up to 1% at heads up to 128 and 1 to 2% past it (6 prompts of 50-700
+// tokens at 16 x 96, 4 layers: 224.1 -> 224.9 us; 300 tokens at 8 x 160, 6 layers:
+// 390 -> 395; the worst measured, one token at 8 x 160, 6 layers: 86.8 -> 91.3).
+template <int HD, bool APPEND>
+__device__ __forceinline__ void prefill_row_fp32(const PrefillLaunch& a, int at, int hd) {
+    constexpr int COLS = (HD + 63) / 64;
+    const int lane = __lane_id();
+    // (found again, so that nothing of it is held through the kernel)
+    asm volatile("" ::: "memory");
+    const int h = blockIdx.x % a.n_heads, item = blockIdx.x / a.n_heads;
+    const int seq = a.work[2 * item], row = a.work[2 * item + 1] + at;
+    const int start = a.start_pos[seq], pos = start + row;
+    const int32_t* trow = a.tables + (size_t)seq * a.max_pages;
+    const size_t col0 = (size_t)(h / a.kv_mul) * hd;
+    const size_t qat = (size_t)(a.row_off[seq] + row) * a.n_heads * hd + (size_t)h * hd;
+    // a key's row of the head; null on a page outside the pool (a row of zeros)
+    auto row_of = [&](const float* pool, const float* fresh, int key) -> const float* {
+        const int page = trow[key >> 4];
+        if ((unsigned)page >= (unsigned)a.num_pages) return nullptr;
+        if (APPEND && key >= start) return fresh + (size_t)(a.row_off[seq] + key - start) * a.kv_dim + col0;
+        return pool + a.layer_off + (size_t)page * a.page_stride + (size_t)(key & 15) * a.kv_dim + col0;
+    };
+    float m = -INFINITY, l = 0.0f, o[COLS] = {};
+#pragma unroll 1
+    for (int key0 = 0; key0 <= pos; key0 += 64) {
+        const int n = min(64, pos - key0 + 1);
+        float s = -INFINITY;
+        if (lane < n) {
+            const float* kr = row_of(a.k_pool, a.k_new, key0 + lane);
+            s = 0.0f;
+            if (kr) {
+#pragma unroll 1
+                for (int d = 0; d < hd; d += 4) {
+                    const float4 k = *reinterpret_cast<const float4*>(kr + d);
+                    const float4 q = *reinterpret_cast<const float4*>(a.q + qat + d);
+                    s = fmaf(q.x * a.qscale, k.x, s);
+                    s = fmaf(q.y * a.qscale, k.y, s);
+                    s = fmaf(q.z * a.qscale, k.z, s);
+                    s = fmaf(q.w * a.qscale, k.w, s);
+                }
+            }
+        }
+        float m_new = fmaxf(m, s);
+#pragma unroll
+        for (int msk = 32; msk > 0; msk >>= 1) m_new = fmaxf(m_new, __shfl_xor(m_new, msk));
+        const float alpha = scale_of(m, m_new);
+        const float p = s == -INFINITY ? 0.0f : exp2f(s - m_new);
+        float psum = p;
+#pragma unroll
+        for (int msk = 32; msk > 0; msk >>= 1) psum += __shfl_xor(psum, msk);
+        l = l * alpha + psum;
+#pragma unroll
+        for (int e = 0; e < COLS; e++) o[e] *= alpha;
+#pragma unroll 1
+        for (int j = 0; j < n; j++) {
+            const float* vr = row_of(a.v_pool, a.v_new, key0 + j);
+            const float pj = __shfl(p, j);
+#pragma unroll
+            for (int e = 0; e < COLS; e++) {
+                const int d = lane + 64 * e;
+                o[e] = fmaf(pj, vr && d < hd ? vr[d] : 0.0f, o[e]);
+            }
+        }
+        m = m_new;
+    }
+#pragma unroll
+    for (int e = 0; e < COLS; e++)
+        if (lane + 64 * e < hd) a.out[qat + lane + 64 * e] = o[e] / l;
+}
+
 // paged_attn_prefill_x3_kernel<HDL, HD, FULL, VP, QT, KSPLIT, BNM, APPEND>: the
 // MFMA kernel's work split and softmax with both products on the bf16 matrix
 // cores at fp32 accuracy.  Q and K are each split into three bf16 parts (hi,
@@ -1123,14 +1200,33 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
             m = mm;
         }
     }
-    if (row < qcount) {
-        const float inv = 1.0f / lsum;
+    const float inv = 1.0f / lsum;
+    uint32_t nan_rows = 0;  // VP 3: of the wave's 16 rows, those with a NaN output
+    if constexpr (VP == 3) {
+        // NaN where an output is NaN (or infinite): 0 times it
+        f32x4 z = {inv * 0.0f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int n = 0; n < NB; n++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) z[i] = fmaf(acc[n][i], 0.0f, z[i]);
+        const bool is_nan = __builtin_isnan((z[0] + z[1]) + (z[2] + z[3]));
+        const uint64_t lanes = __builtin_amdgcn_ballot_w64(is_nan && row < qcount);
+        const uint32_t half = (uint32_t)lanes | (uint32_t)(lanes >> 32);
+        nan_rows = (half | half >> 16) & 0xffffu;
+    }
+    if (row < qcount && !((nan_rows >> ql) & 1)) {
         float* op = a.out + qrow * dim + (size_t)h * hd;
 #pragma unroll
         for (int n = 0; n < NB; n++)
             if (FULL || 16 * n + 4 * g < hd)
                 *reinterpret_cast<float4*>(op + 16 * n + 4 * g) =
                     make_float4(acc[n][0] * inv, acc[n][1] * inv, acc[n][2] * inv, acc[n][3] * inv);
+    }
+    if constexpr (VP == 3) {
+        while (nan_rows) {  // wave-uniform
+            prefill_row_fp32<HD, APPEND != 0>(a, __builtin_amdgcn_readfirstlane(row) + __builtin_ctz(nan_rows), hd);
+            nan_rows &= nan_rows - 1;
+        }
     }
 }
 
