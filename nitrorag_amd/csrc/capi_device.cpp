@@ -694,14 +694,14 @@ int nitro_decode_batch_upload(nitro_kvpool* pool, const int32_t* tables, const i
         d.reserve(nt, batch);
         hipStream_t s = as_stream(stream);
         Staging& st = pool->decode_staging;
-        int32_t* h = st.acquire(nt + 2 * (size_t)batch);
-        std::memcpy(h, tables, nt * sizeof(int32_t));
-        std::memcpy(h + nt, positions, batch * sizeof(int32_t));
+        st.acquire(nt + 2 * (size_t)batch, 3);
+        std::memcpy(st.part(d.tables.ptr, nt), tables, nt * sizeof(int32_t));
+        std::memcpy(st.part(d.pos.ptr, batch), positions, batch * sizeof(int32_t));
+        int32_t* h_slots = st.part(d.slots.ptr, batch);
         for (int b = 0; b < batch; b++)  // where each row's K/V goes (the fused RoPE/append reads it)
-            h[nt + batch + b] = tables[(size_t)b * max_pages + positions[b] / BLOCK_SIZE] * BLOCK_SIZE +
-                                positions[b] % BLOCK_SIZE;
-        st.copy(d.words.ptr, h, nt + 2 * (size_t)batch, s);
-        st.finish(s);
+            h_slots[b] = tables[(size_t)b * max_pages + positions[b] / BLOCK_SIZE] * BLOCK_SIZE +
+                         positions[b] % BLOCK_SIZE;
+        st.send(s);
         d.positions.assign(positions, positions + batch);
         find_decode_groups(pool, d, tables, positions, batch, max_pages);
         d.generation++;
@@ -883,18 +883,25 @@ int nitro_prefill_batch_upload(nitro_kvpool* pool, const int32_t* tables, const 
 
         const size_t nt = (size_t)batch * max_pages;
         const size_t n_work = items.size() * 2, n_wide = wide.size() * 2;
-        const size_t need = nt + 3 * (size_t)batch + 2 * (size_t)total + n_work + n_wide;
+        p.tables.reserve(nt);
+        p.d_start.reserve(batch);
+        p.d_len.reserve(batch);
+        p.d_row_off.reserve(batch);
+        p.slots.reserve(total);
+        p.row_pos.reserve(total);
+        p.work.reserve(n_work);
+        p.work_wide.reserve(n_wide);
         hipStream_t s = as_stream(stream);
         Staging& st = pool->prefill_staging;
-        int32_t* h = st.acquire(need);
-        int32_t* h_tables = h;
-        int32_t* h_start = h_tables + nt;
-        int32_t* h_len = h_start + batch;
-        int32_t* h_off = h_len + batch;
-        int32_t* h_slots = h_off + batch;
-        int32_t* h_row_pos = h_slots + total;
-        int32_t* h_work = h_row_pos + total;
-        int32_t* h_wide = h_work + n_work;
+        st.acquire(nt + 3 * (size_t)batch + 2 * (size_t)total + n_work + n_wide, 8);
+        int32_t* h_tables = st.part(p.tables.ptr, nt);
+        int32_t* h_start = st.part(p.d_start.ptr, batch);
+        int32_t* h_len = st.part(p.d_len.ptr, batch);
+        int32_t* h_off = st.part(p.d_row_off.ptr, batch);
+        int32_t* h_slots = st.part(p.slots.ptr, total);
+        int32_t* h_row_pos = st.part(p.row_pos.ptr, total);
+        int32_t* h_work = st.part(p.work.ptr, n_work);
+        int32_t* h_wide = st.part(p.work_wide.ptr, n_wide);
         std::memcpy(h_tables, tables, nt * sizeof(int32_t));
         std::memcpy(h_start, start_pos, batch * sizeof(int32_t));
         std::memcpy(h_len, num_tokens, batch * sizeof(int32_t));
@@ -913,18 +920,7 @@ int nitro_prefill_batch_upload(nitro_kvpool* pool, const int32_t* tables, const 
             h_wide[2 * i] = wide[i].second.first;
             h_wide[2 * i + 1] = wide[i].second.second;
         }
-        // the device arrays lie as they are staged, so one copy fills them all
-        p.words.reserve(need);
-        p.tables.ptr = p.words.ptr;
-        p.d_start.ptr = p.words.ptr + (h_start - h);
-        p.d_len.ptr = p.words.ptr + (h_len - h);
-        p.d_row_off.ptr = p.words.ptr + (h_off - h);
-        p.slots.ptr = p.words.ptr + (h_slots - h);
-        p.row_pos.ptr = p.words.ptr + (h_row_pos - h);
-        p.work.ptr = p.words.ptr + (h_work - h);
-        p.work_wide.ptr = p.words.ptr + (h_wide - h);
-        st.copy(p.words.ptr, h, need, s);
-        st.finish(s);
+        st.send(s);
         p.start_pos.assign(start_pos, start_pos + batch);
         p.num_tokens.assign(num_tokens, num_tokens + batch);
         p.row_off = row_off;

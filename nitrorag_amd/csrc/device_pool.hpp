@@ -60,14 +60,17 @@ struct DeviceBuffer {
     }
 };
 
-// n words from pinned host memory, read by the kernel over the host link
-// (kv_append.hip).
-hipError_t launch_upload_words(int32_t* dst, const int32_t* pinned, size_t n, hipStream_t stream);
-
-// A part of a DeviceBuffer that holds several arrays of one upload.
-struct DeviceWords {
-    int32_t* ptr = nullptr;
+// The arrays of one upload: array p is words[p] words from word 4 * first[p] of
+// pinned host memory (each starts on 16 bytes), bound for dst[p].
+struct UploadParts {
+    static constexpr int MAX = 8;
+    int32_t* dst[MAX];
+    size_t words[MAX], first[MAX];
+    int count;
 };
+
+// They go by one kernel that reads them over the host link (kv_append.hip).
+hipError_t launch_upload_parts(const UploadParts& parts, const int32_t* pinned, hipStream_t stream);
 
 // Pinned host staging for uploads: reused once the copies that read it have
 // completed (tracked with an event), so callers may free their arrays at once.
@@ -84,12 +87,15 @@ struct Staging {
         if (host) (void)hipHostFree(host);
         if (done) (void)hipEventDestroy(done);
     }
-    int32_t* acquire(size_t n) {
+    // Room for the arrays of one upload, `words` in all and at most `arrays` of
+    // them, added with part().
+    void acquire(size_t words, size_t arrays) {
         if (!done) hip_check(hipEventCreateWithFlags(&done, hipEventDisableTiming), "hipEventCreate");
         if (pending) {
             hip_check(hipEventSynchronize(done), "hipEventSynchronize");
             pending = false;
         }
+        const size_t n = words + 3 * arrays;  // each array starts on 16 bytes
         if (n > count || !host) {
             const size_t cap = grown_capacity(n, count);
             if (host) hip_check(hipHostFree(host), "hipHostFree");
@@ -98,20 +104,39 @@ struct Staging {
             hip_check(hipHostMalloc((void**)&host, cap * sizeof(int32_t)), "hipHostMalloc");
             count = cap;
         }
-        return host;
+        parts.count = 0;
+        used = 0;
     }
-    // Uploads of up to 256 KB (a batch's tables, positions and work lists) go by
-    // a kernel that reads the staging memory: in the stream it costs a launch,
-    // where a copy waits for another engine on both sides (a decode batch's
-    // three copies: 25 us of GPU time between a pass's kernels).
-    void copy(int32_t* dst, const int32_t* src, size_t n, hipStream_t s) {
-        if (n <= 65536) {
-            hip_check(launch_upload_words(dst, src, n, s), "upload launch");
-            return;
+    // Where the next array of the upload, n words for dst, is to be written.
+    int32_t* part(int32_t* dst, size_t n) {
+        int32_t* at = host + used;
+        parts.dst[parts.count] = dst;
+        parts.words[parts.count] = n;
+        parts.first[parts.count++] = used / 4;
+        used += (n + 3) / 4 * 4;
+        return at;
+    }
+    // Uploads of up to 2 MB (a batch's tables, positions and work lists) go by a
+    // kernel that reads the staging memory: in the stream it costs a launch, where
+    // a copy waits for another engine on both sides (a decode batch's three copies:
+    // 25 us of GPU time between a pass's kernels; 16 and 32 prompts of 4096 tokens,
+    // 0.5 and 1.1 MB in eight copies: 202 and 376 us with the host's part, 192 and
+    // 367 by the kernel).
+    void send(hipStream_t s) {
+        if (used <= 1u << 19) {
+            hip_check(launch_upload_parts(parts, host, s), "upload launch");
+        } else {
+            for (int p = 0; p < parts.count; p++)
+                hip_check(hipMemcpyAsync(parts.dst[p], host + 4 * parts.first[p], parts.words[p] * sizeof(int32_t),
+                                         hipMemcpyHostToDevice, s),
+                          "hipMemcpyAsync");
         }
-        hip_check(hipMemcpyAsync(dst, src, n * sizeof(int32_t), hipMemcpyHostToDevice, s),
-                  "hipMemcpyAsync");
+        finish(s);
     }
+
+   private:
+    UploadParts parts{};
+    size_t used = 0;  // words staged
     void finish(hipStream_t s) {
         hip_check(hipEventRecord(done, s), "hipEventRecord");
         pending = true;
@@ -133,14 +158,14 @@ struct DecodeBatch {
     std::vector<uint32_t> page_mark, page_multi;  // per pool page: upload stamps (shared-page scan)
     uint32_t stamp = 0;
     uint64_t generation = 0;         // bumped by every new batch (work-list cache key)
-    DeviceBuffer<int32_t> words;     // tables, pos and slots, one upload
-    DeviceWords tables, pos;
-    DeviceWords slots;               // per row: page * 16 + position % 16 (where its K/V row goes)
+    // Buffers of their own: a captured launch keeps its pointers through uploads
+    // of other shapes.
+    DeviceBuffer<int32_t> tables, pos;
+    DeviceBuffer<int32_t> slots;     // per row: page * 16 + position % 16 (where its K/V row goes)
     void reserve(size_t table_words, size_t rows) {
-        words.reserve(table_words + 2 * rows);
-        tables.ptr = words.ptr;
-        pos.ptr = tables.ptr + table_words;
-        slots.ptr = pos.ptr + rows;
+        tables.reserve(table_words);
+        pos.reserve(rows);
+        slots.reserve(rows);
     }
     // The decode work list last built for this batch, and what it was built for
     // (work_items = 0: longer than the kernel arguments hold).
@@ -168,14 +193,13 @@ struct DecodeBatch {
 struct PrefillBatch {
     int32_t batch = 0, max_pages = 0, total_rows = 0, max_tokens = 0;
     std::vector<int32_t> start_pos, num_tokens, row_off;
-    DeviceBuffer<int32_t> words;      // the arrays below, one upload
-    DeviceWords tables, d_start, d_len, d_row_off;
-    DeviceWords slots;                // per packed row: page*16 + row-in-page
-    DeviceWords row_pos;              // per packed row: its position in the sequence
-    DeviceWords work;                 // per work item: (seq, first query) pairs
+    DeviceBuffer<int32_t> tables, d_start, d_len, d_row_off;
+    DeviceBuffer<int32_t> slots;      // per packed row: page*16 + row-in-page
+    DeviceBuffer<int32_t> row_pos;    // per packed row: its position in the sequence
+    DeviceBuffer<int32_t> work;       // per work item: (seq, first query) pairs
     int32_t work_items = 0;
     int32_t work_block_m = 0;         // query rows per work item the list was built for
-    DeviceWords work_wide;            // the same for items of PREFILL_WIDE_ROWS rows
+    DeviceBuffer<int32_t> work_wide;  // the same for items of PREFILL_WIDE_ROWS rows
     int32_t work_items_wide = 0;
     int32_t max_pos = 0;              // largest position of any row
     // No table entry but a chunk row's own names the page that row lands on:

@@ -165,23 +165,38 @@ hipError_t launch_kv_scatter_rows(float* k_pool, float* v_pool, const float* k, 
 }
 
 namespace {
-// 16 bytes per thread, the last few words one each; grid-stride not needed (the
-// caller's n is bounded by the upload limit).
-__global__ __launch_bounds__(256) void upload_words_kernel(int32_t* __restrict__ dst, const int32_t* __restrict__ src,
-                                                           int n) {
+// 16 bytes per thread (an array's last words: as many as it has; the staging memory
+// is padded to 16 bytes).
+__global__ __launch_bounds__(256) void upload_parts_kernel(UploadParts parts, const int4* __restrict__ src, int n) {
     const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n / 4)
-        reinterpret_cast<int4*>(dst)[i] = reinterpret_cast<const int4*>(src)[i];
-    else if (i - n / 4 < n % 4)
-        dst[n / 4 * 4 + i - n / 4] = src[n / 4 * 4 + i - n / 4];
+    const int4 v = src[min(i, n - 1)];
+    int32_t* dst = parts.dst[0];
+    int words = (int)parts.words[0], first = 0;
+#pragma unroll
+    for (int k = 1; k < UploadParts::MAX; k++)
+        if (k < parts.count && i >= (int)parts.first[k])
+            dst = parts.dst[k], words = (int)parts.words[k], first = (int)parts.first[k];
+    const int w = 4 * (i - first);  // this thread's first word of the array
+    if (w + 4 <= words) {
+        *reinterpret_cast<int4*>(dst + w) = v;
+    } else {
+        if (w < words) dst[w] = v.x;
+        if (w + 1 < words) dst[w + 1] = v.y;
+        if (w + 2 < words) dst[w + 2] = v.z;
+    }
 }
 }  // namespace
 
-hipError_t launch_upload_words(int32_t* dst, const int32_t* pinned, size_t n, hipStream_t stream) {
+hipError_t launch_upload_parts(const UploadParts& parts, const int32_t* pinned, hipStream_t stream) {
+    if (parts.count == 0) return hipSuccess;
+    const int last = parts.count - 1;
+    const size_t n = parts.first[last] + (parts.words[last] + 3) / 4;  // 16-byte units
+    uintptr_t align = (uintptr_t)pinned;
+    for (int p = 0; p < parts.count; p++) align |= (uintptr_t)parts.dst[p];
+    if (n > (1u << 28) || align % 16) return hipErrorInvalidValue;
     if (n == 0) return hipSuccess;
-    if (n > (1u << 30) || ((uintptr_t)dst | (uintptr_t)pinned) % 16) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(upload_words_kernel, dim3((unsigned)((n / 4 + 3 + 255) / 256)), dim3(256), 0, stream, dst, pinned,
-                       (int)n);
+    hipLaunchKernelGGL(upload_parts_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, parts,
+                       reinterpret_cast<const int4*>(pinned), (int)n);
     return hipGetLastError();
 }
 

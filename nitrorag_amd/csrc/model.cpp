@@ -106,10 +106,9 @@ void upload_tokens(nitro_model* m, const int32_t* tokens, int rows, hipStream_t 
     for (int i = 0; i < rows; i++)
         if (tokens[i] < 0 || tokens[i] >= m->vocab)
             throw Error(ERR_INVALID_ARGUMENT, "token id " + std::to_string(tokens[i]) + " outside the vocabulary");
-    int32_t* h = m->staging.acquire(rows);
-    std::memcpy(h, tokens, sizeof(int32_t) * rows);
-    m->staging.copy(m->tokens.ptr, h, rows, s);
-    m->staging.finish(s);
+    m->staging.acquire(rows, 1);
+    std::memcpy(m->staging.part(m->tokens.ptr, rows), tokens, sizeof(int32_t) * rows);
+    m->staging.send(s);
 }
 
 // logits = wcls . rms_norm(x) for `rows` rows of the residual stream x, which

@@ -223,15 +223,14 @@ int nitro_sched_step(nitro_scheduler* sched, nitro_model* model, nitro_kvpool* p
         // other entries, the chunk's table.
         const size_t n_in = (size_t)P + B + desc.size() + other.size() + chunk_table.size();
         d.step_in.reserve(n_in);
-        int32_t* hin = d.staging.acquire(n_in);
-        int32_t* w = hin;
+        d.staging.acquire(n_in, 1);
+        int32_t* w = d.staging.part(d.step_in.ptr, n_in);
         w = std::copy(p.prefill_tokens.begin(), p.prefill_tokens.end(), w);
         w = std::copy(p.decode_tokens.begin(), p.decode_tokens.end(), w);
         w = std::copy(desc.begin(), desc.end(), w);
         w = std::copy(other.begin(), other.end(), w);
         std::copy(chunk_table.begin(), chunk_table.end(), w);
-        d.staging.copy(d.step_in.ptr, hin, n_in, s);
-        d.staging.finish(s);
+        d.staging.send(s);
         const int32_t* d_tokens = d.step_in.ptr;
         const int32_t* d_desc = d.step_in.ptr + P + B;
         const int32_t* d_other = d_desc + desc.size();
