@@ -101,7 +101,9 @@ struct Staging {
             if (host) hip_check(hipHostFree(host), "hipHostFree");
             host = nullptr;
             count = 0;
-            hip_check(hipHostMalloc((void**)&host, cap * sizeof(int32_t)), "hipHostMalloc");
+            // Coherent by request, not by the runtime's default (HIP_HOST_COHERENT): a
+            // kernel reads the same addresses again with every upload.
+            hip_check(hipHostMalloc((void**)&host, cap * sizeof(int32_t), hipHostMallocCoherent), "hipHostMalloc");
             count = cap;
         }
         parts.count = 0;
