@@ -131,14 +131,12 @@ __global__ __launch_bounds__(64 * GEMM_WAVES, GEMM_NT == 8 ? 2 : 3) void q8_gemm
                       : ((uint32_t)min(b0 + 16 * m + lr, batch - 1) * n + 8 * lg) * 4;
     constexpr uint32_t XSTEP = PRE ? Q8_SPLIT_BYTES : Q8_BLOCK * 4;
 
-    // Row-major x: workgroups start their walk over the blocks at different
-    // blocks.  Rows are often a multiple of 4 KB apart, so a block of them sits
-    // on one L2 channel, and workgroups in step would all wait on the same one.
-    const int start = PRE ? 0 : wg * 2 % nb;
-    auto walk = [&](int i) __attribute__((always_inline)) {  // the i-th block (past the end: the last)
-        const int b = min(i, nb - 1) + start;
-        return b < nb ? b : b - nb;
-    };
+    // The i-th block (past the end: the last).  Every workgroup walks the blocks in
+    // the same order, so equal rows give equal bits wherever they lie.  (Starting
+    // at different blocks for row-major x, whose rows sit on one L2 channel when
+    // they are a multiple of 4 KB apart, gained 1.2% at 192 and 256 rows of 4096 x
+    // 11008 and lost up to 1.9% elsewhere.)
+    auto walk = [&](int i) __attribute__((always_inline)) { return min(i, nb - 1); };
     // A block's loads.  None is behind a branch (a block past the end rereads
     // the last), so that each wait counts exactly the loads it needs.
     struct WRound {
@@ -260,15 +258,32 @@ __global__ __launch_bounds__(64 * GEMM_WAVES, GEMM_NT == 8 ? 2 : 3) void q8_gemm
             }
         }
     };
-    auto flush = [&](bool first) __attribute__((always_inline)) {
+    // The last two tiles' sums into their accumulators.
+    auto scale_late = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int m = 0; m < GEMM_MT; m++)
 #pragma unroll
-            for (int t = 0; t < GEMM_NT; t++) {
+            for (int u = 0; u < 2; u++) {
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    acc[m][GEMM_NT - 2 + u][i] = fmaf(late_sc[u], late[m][u][i], acc[m][GEMM_NT - 2 + u][i]);
+                late[m][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+        late_sc[0] = late_sc[1] = 0.f;
+    };
+    // (late sums included, after the other tiles: every tile's chains hold the
+    // same blocks)
+    auto flush = [&](bool first) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < GEMM_NT; t++) {
+            if (t == GEMM_NT - 2) scale_late();
+#pragma unroll
+            for (int m = 0; m < GEMM_MT; m++) {
                 f32x4& slot = sums[wave][m * GEMM_NT + t][lane];
                 slot = first ? acc[m][t] : slot + acc[m][t];
                 acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
             }
+        }
     };
     WRound wa, wb;
     XRound xa, xb;
@@ -299,13 +314,7 @@ __global__ __launch_bounds__(64 * GEMM_WAVES, GEMM_NT == 8 ? 2 : 3) void q8_gemm
         step(blk + 1, xb, xa, wb);
     }
     if (blk < nb) step(blk, xa, xb, wa);
-#pragma unroll
-    for (int m = 0; m < GEMM_MT; m++)
-#pragma unroll
-        for (int u = 0; u < 2; u++)
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-                acc[m][GEMM_NT - 2 + u][i] = fmaf(late_sc[u], late[m][u][i], acc[m][GEMM_NT - 2 + u][i]);
+    scale_late();
     if (nb >= GEMM_FLUSH) {
 #pragma unroll
         for (int m = 0; m < GEMM_MT; m++)

@@ -66,3 +66,18 @@ def test_layer_of_many_rows():
     check_logits(got, want, "layer of many rows")
     for g, r in ((dk, k), (dv, v)):
         assert np.abs(g.cpu().numpy() - r).max() <= 1e-4 + 1e-3 * np.abs(r).max()
+
+
+@pytest.mark.parametrize("n,d,batch", [(2080, 8200, 400), (4096, 4200, 1000)])
+def test_equal_rows_give_equal_bits(n, d, batch):
+    """Activation rows that are the same, in any panel, and weight rows that are the
+    same, in any column tile, give the same bits: an output's sums are added in an
+    order that depends on n alone."""
+    print(f"q8 equal rows n {n} d {d} batch {batch}", flush=True)
+    rng = np.random.default_rng(n)
+    q = rng.integers(-127, 128, (5, n // 32, 32)).astype(np.int8)
+    scale = (rng.random((5, n // 32)) * 0.02 + 1e-3).astype(np.float32)
+    few = np.concatenate((scale[..., None].view(np.uint8), q.view(np.uint8)), axis=-1).reshape(5, -1)
+    x = rng.standard_normal((7, n)).astype(np.float32)
+    got = run_gpu(few[np.arange(d) % 5].reshape(-1), x[np.arange(batch) % 7], d, 0)
+    assert np.array_equal(got, got[:7, :5][np.arange(batch) % 7][:, np.arange(d) % 5])
