@@ -31,8 +31,10 @@ struct nitro_model {
     uint8_t* tiled = nullptr;
     size_t tiled_bytes = 0;
     size_t t_wq = 0, t_wk = 0, t_wv = 0, t_wo = 0, t_w1 = 0, t_w2 = 0, t_w3 = 0;
-    DeviceBuffer<float> x, attn, q, hb, last, ss;
-    DeviceBuffer<uint8_t> xsplit, hsplit;  // x (times the next norm's weights) and hb in split form
+    DeviceBuffer<float> x, attn, q, last, ss;
+    DeviceBuffer<uint8_t> hb;      // SwiGLU's output: as floats, or in split form
+    DeviceBuffer<uint8_t> xsplit;  // x (times the next norm's weights) in split form
+    int max_rows = 0;              // of any forward
     DeviceBuffer<int32_t> tokens;
     Staging staging;
 
@@ -80,18 +82,27 @@ void ensure_tiled(nitro_model* m, hipStream_t s) {
     m->tiled = t;
 }
 
-void reserve_rows(nitro_model* m, int rows) {
-    const size_t r = (size_t)rows;
+// Room for a forward of `rows` rows.  A model that has run no full-row products of
+// more than 4 rows holds nothing in split form; one that has holds hb once, in the
+// larger of its two forms, for as many rows as any forward had.
+void reserve_rows(nitro_model* m, int rows, bool last_block) {
+    m->max_rows = std::max(m->max_rows, rows);
+    const size_t r = (size_t)m->max_rows;
     m->x.reserve(r * m->dim);
     m->attn.reserve(r * m->dim);
     m->ss.reserve(r * (size_t)((m->dim + 15) / 16));
     m->q.reserve(r * m->dim);
-    m->hb.reserve(r * m->hidden);
     m->tokens.reserve(r);
-    if (q8_split_usable(r, m->dim, m->hidden)) {
-        m->xsplit.reserve(q8_split_bytes(r, m->dim));
-        m->hsplit.reserve(q8_split_bytes(r, (size_t)std::max(m->dim, m->hidden)));
+    size_t hb_bytes = r * m->hidden * sizeof(float);
+    if (m->tiled || (!last_block && rows > Q8_GEMV_MAX_BATCH)) {
+        const size_t sr = q8_split_usable(r, m->dim, m->hidden) ? r : (size_t)rows;
+        if (q8_split_usable(sr, m->dim, m->hidden)) {
+            if (!m->xsplit.ptr) m->hb.reset();  // its one change of form: to the size, not to twice it
+            m->xsplit.reserve(q8_split_bytes(sr, m->dim));
+            hb_bytes = std::max(hb_bytes, q8_split_bytes(sr, (size_t)std::max(m->dim, m->hidden)));
+        }
     }
+    m->hb.reserve(hb_bytes);
 }
 
 void check_model_pool(const nitro_model* m, const nitro_kvpool* pool) {
@@ -144,7 +155,8 @@ void layers(nitro_model* m, nitro_kvpool* pool, const int32_t* tokens, int rows,
     // the launch that made them.
     const bool use_split = !last && q8_split_usable(rows, dim, hid);
     char* const xs = reinterpret_cast<char*>(use_split ? m->xsplit.ptr : nullptr);
-    char* const hs = reinterpret_cast<char*>(use_split ? m->hsplit.ptr : nullptr);
+    char* const hs = reinterpret_cast<char*>(use_split ? m->hb.ptr : nullptr);
+    float* const hb = reinterpret_cast<float*>(m->hb.ptr);
     auto x_out = [&](const float* next_norm) { return next_norm ? Q8SplitOut{xs, next_norm, dim / 32} : Q8SplitOut{}; };
     hip_check(launch_embed_rows(m->f32(m->o_emb), tokens, m->x.ptr, rows, dim, m->vocab, pool->bad_pages.ptr,
                                 m->ss.ptr, use_split ? x_out(m->f32(m->o_rms_att)) : Q8SplitOut{}, s),
@@ -176,11 +188,11 @@ void layers(nitro_model* m, nitro_kvpool* pool, const int32_t* tokens, int rows,
         t13.w[0] = m->q8t(m->t_w1, l, hid, dim);
         t13.w[1] = m->q8t(m->t_w3, l, hid, dim);
         hip_check(launch_q8_swiglu(m->q8(m->o_w1, l, hid, dim), m->q8(m->o_w3, l, hid, dim), m->x.ptr,
-                                   m->hb.ptr, rows, dim, hid, last, ffn, s, t13,
+                                   hb, rows, dim, hid, last, ffn, s, t13,
                                    Q8Split{xs, Q8SplitOut{hs, nullptr, hid / 32}, nullptr}),
                   "q8_swiglu launch");
         // x += w2 . hb (:682-684)
-        hip_check(launch_q8_residual(m->q8(m->o_w2, l, dim, hid), m->hb.ptr, m->x.ptr, m->ss.ptr, rows, hid,
+        hip_check(launch_q8_residual(m->q8(m->o_w2, l, dim, hid), hb, m->x.ptr, m->ss.ptr, rows, hid,
                                      dim, last, s, m->q8t(m->t_w2, l, dim, hid),
                                      Q8Split{hs, use_split && l + 1 < m->n_layers ? x_out(att.weight + dim) : Q8SplitOut{}, nullptr}),
                   "q8 w2 launch");
@@ -257,7 +269,7 @@ void forward_mixed(nitro_model* m, nitro_kvpool* pool, const int32_t* tokens, in
     const Q8Rope rope = prefill_as_decode || P == 0
                             ? rope_args(m, pool, d.pos.ptr, d.slots.ptr, P + B, nullptr, nullptr)
                             : rope_args(m, pool, pf.row_pos.ptr, pf.slots.ptr, P, d.pos.ptr, d.slots.ptr);
-    reserve_rows(m, P + B);
+    reserve_rows(m, P + B, semantics == NITRO_Q8_LAST_BLOCK);
     layers(m, pool, tokens, P + B, semantics, rope, s, [&](int l) {
         if (prefill_as_decode) {
             // every row attends its own prefix (keys 0..position) in one
@@ -395,7 +407,7 @@ int nitro_forward_decode_batch(nitro_model* m, nitro_kvpool* pool, const int32_t
         hipStream_t s = as_stream(stream);
         const DecodeBatch& d = pool->decode;
         check_positions(m, max_of(d.positions));
-        reserve_rows(m, batch);
+        reserve_rows(m, batch, semantics == NITRO_Q8_LAST_BLOCK);
         upload_tokens(m, tokens, batch, s);
         const Q8Rope rope = rope_args(m, pool, d.pos.ptr, d.slots.ptr, batch, nullptr, nullptr);
         layers(m, pool, m->tokens.ptr, batch, semantics, rope, s, [&](int l) {
@@ -421,7 +433,7 @@ int nitro_forward_prefill(nitro_model* m, nitro_kvpool* pool, const int32_t* tok
         require(total_rows == p.total_rows, ERR_INVALID_ARGUMENT,
                 "total_rows differs from the uploaded prefill batch");
         hipStream_t s = as_stream(stream);
-        reserve_rows(m, total_rows);
+        reserve_rows(m, total_rows, semantics == NITRO_Q8_LAST_BLOCK);
         m->last.reserve((size_t)p.batch * m->dim);
         upload_tokens(m, tokens, total_rows, s);
         check_positions(m, p.max_pos);
