@@ -51,10 +51,13 @@ constexpr int GEMM_FLUSH = 8;
 // The 16-byte run c (8 k) of a row in an LDS weight buffer (64 bytes a row).
 __device__ __forceinline__ int w_at(int row, int c) { return row * 32 + ((c ^ (row >> 1)) & 3) * 8; }
 
-template <Q8Epilogue EPI, bool TILED, bool PRE, int GEMM_NT>
+// A model's launches (all but Store) read its matrices in the tile layout and x in
+// split form (PRE); q8_matmul's have neither.
+template <Q8Epilogue EPI, int GEMM_NT>
 __global__ __launch_bounds__(64 * GEMM_WAVES, GEMM_NT == 8 ? 2 : 3) void q8_gemm_kernel(Q8Group grp, const void* __restrict__ xin,
                                                                      int batch, int n, int col_tiles, Q8Norm nm, Q8Resid resid,
                                                                      Q8SplitOut out, Q8Rope rope) {
+    constexpr bool TILED = EPI != Q8Epilogue::Store, PRE = TILED;
     constexpr int GEMM_BN = 16 * GEMM_NT;
     constexpr bool NORM = EPI == Q8Epilogue::SwiGlu || EPI == Q8Epilogue::Rope;
     constexpr bool SWIGLU = EPI == Q8Epilogue::SwiGlu;
@@ -481,15 +484,11 @@ __global__ __launch_bounds__(256) void q8_split_kernel(const float* __restrict__
     }
 }
 
-template <Q8Epilogue EPI, bool PRE, int NT>
-void launch(bool tiled, dim3 grid, hipStream_t stream, const Q8Group& grp, const void* x, int batch, int n, int cols,
+template <Q8Epilogue EPI, int NT>
+void launch(dim3 grid, hipStream_t stream, const Q8Group& grp, const void* x, int batch, int n, int cols,
             const Q8Norm& nm, const Q8Resid& resid, const Q8SplitOut& out, const Q8Rope& rope) {
-    if (tiled)
-        hipLaunchKernelGGL((q8_gemm_kernel<EPI, true, PRE, NT>), grid, dim3(64 * GEMM_WAVES), 0, stream, grp, x, batch,
-                           n, cols, nm, resid, out, rope);
-    else
-        hipLaunchKernelGGL((q8_gemm_kernel<EPI, false, PRE, NT>), grid, dim3(64 * GEMM_WAVES), 0, stream, grp, x, batch,
-                           n, cols, nm, resid, out, rope);
+    hipLaunchKernelGGL((q8_gemm_kernel<EPI, NT>), grid, dim3(64 * GEMM_WAVES), 0, stream, grp, x, batch, n, cols, nm,
+                       resid, out, rope);
 }
 
 }  // namespace
@@ -505,6 +504,7 @@ bool launch_q8_gemm(Q8Epilogue epilogue, const Q8Group& grp, const float* x, con
     }
     if (q8_tiled_bytes(dmax, n) >= (1ull << 32) || q8_split_bytes(batch, n) >= (1ull << 32)) return false;
     const bool pre = epilogue != Q8Epilogue::Store;
+    if (pre && !tiled) return false;
     if (pre && !split.in && (!split.scratch || nm.weight)) return false;
     if (epilogue == Q8Epilogue::SwiGlu && !split.out.planes) return false;
     auto columns = [&](int bn) {  // column tiles of bn weight rows
@@ -548,10 +548,10 @@ bool launch_q8_gemm(Q8Epilogue epilogue, const Q8Group& grp, const float* x, con
     const auto run = [&](auto nt) {
         constexpr int NT = decltype(nt)::value;
         switch (epilogue) {
-            case Q8Epilogue::Store: launch<Q8Epilogue::Store, false, NT>(tiled, grid, stream, grp, in, batch, n, cols, nm, resid, split.out, rope); break;
-            case Q8Epilogue::Residual: launch<Q8Epilogue::Residual, true, NT>(tiled, grid, stream, grp, in, batch, n, cols, nm, resid, split.out, rope); break;
-            case Q8Epilogue::SwiGlu: launch<Q8Epilogue::SwiGlu, true, NT>(tiled, grid, stream, grp, in, batch, n, cols, nm, resid, split.out, rope); break;
-            case Q8Epilogue::Rope: launch<Q8Epilogue::Rope, true, NT>(tiled, grid, stream, grp, in, batch, n, cols, nm, resid, split.out, rope); break;
+            case Q8Epilogue::Store: launch<Q8Epilogue::Store, NT>(grid, stream, grp, in, batch, n, cols, nm, resid, split.out, rope); break;
+            case Q8Epilogue::Residual: launch<Q8Epilogue::Residual, NT>(grid, stream, grp, in, batch, n, cols, nm, resid, split.out, rope); break;
+            case Q8Epilogue::SwiGlu: launch<Q8Epilogue::SwiGlu, NT>(grid, stream, grp, in, batch, n, cols, nm, resid, split.out, rope); break;
+            case Q8Epilogue::Rope: launch<Q8Epilogue::Rope, NT>(grid, stream, grp, in, batch, n, cols, nm, resid, split.out, rope); break;
         }
     };
     if (narrow)

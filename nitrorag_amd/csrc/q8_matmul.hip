@@ -1208,10 +1208,11 @@ struct MmaRound {
     u32x4 x[BT][U][PRE ? 3 : 2];  // PRE: hi, mid, lo; else 8 floats
 };
 
-template <int NMAT, int BT, bool TILED, bool PRE, bool NT, bool SWIGLU, bool NORM, bool RESID, bool ROPE>
+template <int NMAT, int BT, bool PRE, bool NT, bool SWIGLU, bool NORM, bool RESID, bool ROPE>
 __global__ __launch_bounds__(64 * MMA_WAVES) void q8_mma_kernel(Q8Group grp, const void* __restrict__ xin,
                                                                 int batch, int n, Q8Norm nm, Q8Resid resid,
                                                                 Q8SplitOut out, Q8Rope rope) {
+    constexpr bool TILED = NORM || RESID;  // a model's launches read its tile layout
     constexpr int U = mma_unroll<NMAT, BT>();
     constexpr int STRIDE = MMA_WAVES * U;  // blocks per round of the workgroup
     __shared__ float red[MMA_WAVES][NMAT][16 * MMA_TILE_STRIDE];
@@ -1526,7 +1527,7 @@ void launch_gemv(const Q8Group& grp, const float* x, int n, int dmax, const Q8No
                        rs, rp);
 }
 
-template <int NMAT, bool TILED, bool PRE, bool SWIGLU, bool NORM, bool RESID, bool ROPE>
+template <int NMAT, bool PRE, bool SWIGLU, bool NORM, bool RESID, bool ROPE>
 void launch_mma(const Q8Group& grp, const void* x, int batch, int n, int dmax, const Q8Norm& nm, const Q8Resid& rs,
                 const Q8SplitOut& out, const Q8Rope& rp, hipStream_t stream) {
     const dim3 block(64 * MMA_WAVES);
@@ -1540,7 +1541,7 @@ void launch_mma(const Q8Group& grp, const void* x, int batch, int n, int dmax, c
     // product at batch 32 (256 tiles) took 32.6 us against 25.2 with two.
     const unsigned btiles = (unsigned)((batch + 15) / 16);
     const auto run = [&](auto bt, auto nt, dim3 grid) {
-        hipLaunchKernelGGL((q8_mma_kernel<NMAT, decltype(bt)::value, TILED, PRE, decltype(nt)::value, SWIGLU, NORM, RESID, ROPE>),
+        hipLaunchKernelGGL((q8_mma_kernel<NMAT, decltype(bt)::value, PRE, decltype(nt)::value, SWIGLU, NORM, RESID, ROPE>),
                            grid, block, 0, stream, grp, x, batch, n, nm, rs, out, rp);
     };
     using std::integral_constant;
@@ -1610,20 +1611,16 @@ void launch_group(const Q8Group& grp, const float* x, int batch, int n, int dmax
     if (use_mma() && launch_q8_gemm(EPI, grp, x, split, batch, n, nm, rs, rp, stream)) return;
     const bool mma_fits = mma_offsets_fit(dmax, n, batch, split.in != nullptr) && (size_t)batch * n < (1ull << 32) &&
                           (!NORM || split.in || n <= MMA_NORM_MAX_N);
-    if (use_mma() && mma_fits) {
-        bool tiled = true;
-        for (int m = 0; m < NMAT; m++) tiled = tiled && grp.wt[m] != nullptr;
-        // (a model hands on split activations only where it holds the tile layout)
+    bool layout = true;  // a model's launches: their matrices in the tile layout
+    if constexpr (NORM || RESID)
+        for (int m = 0; m < NMAT; m++) layout = layout && grp.wt[m] != nullptr;
+    if (use_mma() && mma_fits && layout) {
         if constexpr (NORM || RESID)
             if (split.in) {
-                launch_mma<NMAT, true, true, SWIGLU, NORM, RESID, ROPE>(grp, split.in, batch, n, dmax, nm, rs, split.out,
-                                                                        rp, stream);
+                launch_mma<NMAT, true, SWIGLU, NORM, RESID, ROPE>(grp, split.in, batch, n, dmax, nm, rs, split.out, rp, stream);
                 return;
             }
-        if (tiled)
-            launch_mma<NMAT, true, false, SWIGLU, NORM, RESID, ROPE>(grp, x, batch, n, dmax, nm, rs, split.out, rp, stream);
-        else
-            launch_mma<NMAT, false, false, SWIGLU, NORM, RESID, ROPE>(grp, x, batch, n, dmax, nm, rs, split.out, rp, stream);
+        launch_mma<NMAT, false, SWIGLU, NORM, RESID, ROPE>(grp, x, batch, n, dmax, nm, rs, split.out, rp, stream);
         return;
     }
     hipLaunchKernelGGL((q8_matmul_kernel<NMAT, SWIGLU, NORM, RESID, ROPE>), grid, block, 0, stream, grp, x, batch, n,
