@@ -298,6 +298,18 @@ int nitro_rope_kv_append_prefill(nitro_kvpool* pool, int32_t layer, float* q, fl
 int nitro_q8_matmul(const void* w, const float* x, float* out, int32_t batch, int32_t n,
                     int32_t d, int32_t semantics, void* stream);
 
+/* No counterpart in the reference: which kernel takes a full-row product of
+ * `batch` rows on the current device.  *rows is the number of weight rows per
+ * workgroup (64 or 128) where the kernel for many rows takes it, 0 where another
+ * one does.  launch: nitro_q8_matmul's own, or one of a model's: wo / w2 with the
+ * residual add, w1 and w3 with SwiGLU (d rows each), wq, wk and wv (d rows and
+ * twice d_kv; d_kv is read for this one only).  Needs no GPU. */
+#define NITRO_Q8_LAUNCH_MATMUL 0
+#define NITRO_Q8_LAUNCH_RESIDUAL 1
+#define NITRO_Q8_LAUNCH_SWIGLU 2
+#define NITRO_Q8_LAUNCH_QKV 3
+int nitro_q8_tile_rows(int32_t launch, int32_t batch, int32_t n, int32_t d, int32_t d_kv, int32_t* rows);
+
 /* ------------------------ transformer step (model) -------------------------
  * The forward passes of src/model_q8.cpp around the attention path, on the
  * device: embedding, per layer rms_norm -> wq/wk/wv (Q8) -> RoPE + KV append

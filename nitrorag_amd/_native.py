@@ -95,6 +95,7 @@ SIGNATURES = {
     "nitro_rope_kv_append_prefill": [_vp, _i32, _fp, _fp, _fp, _fp, _fp, _i32, _i32, _i32, _i32,
                                      _vp],
     "nitro_q8_matmul": [_vp, _fp, _fp, _i32, _i32, _i32, _i32, _vp],
+    "nitro_q8_tile_rows": [_i32, _i32, _i32, _i32, _i32, _i32p],
     "nitro_model_create": [_vp, ctypes.c_uint64, ctypes.POINTER(_vp)],
     "nitro_model_destroy": [_vp],
     "nitro_model_config": [_vp, _i32p],

@@ -1118,6 +1118,17 @@ int nitro_q8_matmul(const void* w, const float* x, float* out, int32_t batch, in
     });
 }
 
+int nitro_q8_tile_rows(int32_t launch, int32_t batch, int32_t n, int32_t d, int32_t d_kv, int32_t* rows) {
+    return guarded([&] {
+        require(rows != nullptr, ERR_INVALID_ARGUMENT, "null output pointer");
+        require(launch >= NITRO_Q8_LAUNCH_MATMUL && launch <= NITRO_Q8_LAUNCH_QKV, ERR_INVALID_ARGUMENT,
+                "launch must be one of NITRO_Q8_LAUNCH_*");
+        require(batch > 0 && n > 0 && d > 0 && n % 32 == 0 && (launch != NITRO_Q8_LAUNCH_QKV || d_kv > 0),
+                ERR_INVALID_ARGUMENT, "batch, n, d (and d_kv) must be positive, n a multiple of 32");
+        *rows = q8_tile_rows(launch, batch, n, d, d_kv);
+    });
+}
+
 int nitro_kvpool_decode_counts(nitro_kvpool* pool, int64_t* launches, int64_t* shared_prefix_launches) {
     return guarded([&] {
         require_pool(pool);

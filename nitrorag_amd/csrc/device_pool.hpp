@@ -375,6 +375,8 @@ struct Q8Split {
 // Whether the launches of a model with these widths may use split activations
 // at this many rows (32-bit offsets; the bf16 kernels selected).
 bool q8_split_usable(size_t rows, size_t dim, size_t hidden);
+// nitro_q8_tile_rows (q8_gemm.hip).
+int q8_tile_rows(int launch, int batch, int n, int d, int d_kv);
 // tiled = the tile layout of w (rows of BlockQ8, d x n)
 hipError_t launch_q8_tile(const void* w, void* tiled, int d, int n, hipStream_t stream);
 // Q8_0 matrix product (rows of BlockQ8, fp32 activations); last_block_only

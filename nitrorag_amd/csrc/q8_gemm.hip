@@ -493,50 +493,67 @@ void launch(dim3 grid, hipStream_t stream, const Q8Group& grp, const void* x, in
 
 }  // namespace
 
-bool launch_q8_gemm(Q8Epilogue epilogue, const Q8Group& grp, const float* x, const Q8Split& split, int batch, int n,
-                    const Q8Norm& nm, const Q8Resid& resid, const Q8Rope& rope, hipStream_t stream) {
-    const int members = epilogue == Q8Epilogue::Rope ? 3 : epilogue == Q8Epilogue::SwiGlu ? 2 : 1;
-    bool tiled = true;
-    int dmax = 0;
-    for (int m = 0; m < members; m++) {
-        tiled = tiled && grp.wt[m] != nullptr;
-        dmax = std::max(dmax, grp.d[m]);
-    }
-    if (q8_tiled_bytes(dmax, n) >= (1ull << 32) || q8_split_bytes(batch, n) >= (1ull << 32)) return false;
+namespace {
+int members_of(Q8Epilogue e) { return e == Q8Epilogue::Rope ? 3 : e == Q8Epilogue::SwiGlu ? 2 : 1; }
+
+// Column tiles of `rows` weight rows (with SwiGLU, of w1 and w3 in equal parts).
+int columns(Q8Epilogue e, const int* d, int rows) {
+    if (e == Q8Epilogue::SwiGlu) return (d[0] + rows / 2 - 1) / (rows / 2);
+    int c = 0;
+    for (int m = 0; m < members_of(e); m++) c += (d[m] + rows - 1) / rows;
+    return c;
+}
+}  // namespace
+
+int q8_gemm_tile(Q8Epilogue epilogue, const int* d, int batch, int n) {
+    const int members = members_of(epilogue);
     const bool pre = epilogue != Q8Epilogue::Store;
-    if (pre && !tiled) return false;
-    if (pre && !split.in && (!split.scratch || nm.weight)) return false;
-    if (epilogue == Q8Epilogue::SwiGlu && !split.out.planes) return false;
-    auto columns = [&](int bn) {  // column tiles of bn weight rows
-        int c = 0;
-        for (int m = 0; m < members; m++) c += (grp.d[m] + bn - 1) / bn;
-        return epilogue == Q8Epilogue::SwiGlu ? (grp.d[0] + bn / 2 - 1) / (bn / 2) : c;
-    };
+    const int dmax = epilogue == Q8Epilogue::Rope ? std::max(d[0], std::max(d[1], d[2])) : d[0];
+    if (q8_tiled_bytes(dmax, n) >= (1ull << 32) || q8_split_bytes(batch, n) >= (1ull << 32)) return 0;
     // 128 or 64 weight rows per workgroup: whichever fills its dispatch rounds
     // better (two or three workgroups per CU; a round costs about the same
     // however full it is).  wo at 5520 x 768: 264 wide workgroups 51 us, 528
     // narrow 39; at 1600 x 4096, 416 wide ones fit a round and 832 narrow ones
     // do not: 4.20 ms per pass against 4.38.  Where a wave splits x itself, it
-    // does so twice as often with 64 (1024 rows, 4096 x 11008, with scales still
-    // loaded per tile: 2.08 ms against 1.70), hence the 0.75.
-    constexpr int CUS = 256;
+    // does so twice as often with 64, hence the 0.75 (also from an earlier form).
+    const long long cus = device_cus();
     const long long panels = (batch + GEMM_BM - 1) / GEMM_BM;
-    const long long wide = panels * columns(128), slim = panels * columns(64);
-    const long long wide_rounds = (wide + 2 * CUS - 1) / (2 * CUS), slim_rounds = (slim + 3 * CUS - 1) / (3 * CUS);
-    const double wide_fill = (double)wide / (wide_rounds * 2 * CUS), slim_fill = (double)slim / (slim_rounds * 3 * CUS);
+    const long long wide = panels * columns(epilogue, d, 128), slim = panels * columns(epilogue, d, 64);
+    const long long wide_rounds = (wide + 2 * cus - 1) / (2 * cus), slim_rounds = (slim + 3 * cus - 1) / (3 * cus);
+    const double wide_fill = (double)wide / (wide_rounds * 2 * cus), slim_fill = (double)slim / (slim_rounds * 3 * cus);
     const bool narrow = slim_fill * (pre ? 1.0 : 0.75) > wide_fill;
-    const long long wgs = narrow ? slim : wide;
-    // A round takes about 1 us per block (1.3 with 128 rows) at any size, the
-    // small-batch kernel rows x outputs x n / 26.5e6 us, so this kernel pays
-    // from about 830,000 outputs per round.  Three products there and with the
-    // rule: 128 rows at 4096 x 11008 667 / 488 us; 256 rows at 2048 x 5632 344 /
-    // 249, at 4096 x 11008 1325 / 682, at 768 x 2048 58 / 58 (none taken; all of
-    // them taken lost at 768, as 128 rows of w2 at 4096 x 11008 did).
+    // From how many outputs per dispatch round this kernel is taken.  The line was
+    // fitted to an earlier form of it and is cautious for the present one: no
+    // product measured goes to this kernel where the small-batch one is faster, but
+    // the 64-row tile would win sooner and more often.  One product, small-batch /
+    // 64 rows / 128 rows, us (the rule's choice in brackets): 256 rows of 2048 x
+    // 2048 [47] / 42 / 66, of 4096 x 4096 [169] / 84 / 131; 64 rows of 11008 x 4096
+    // [128] / 79 / 128, 128 rows 232 / 84 / [130]; 512 rows of 4096 x 4096 335 / 87 /
+    // [131], of 2048 x 768 [31] / 19 / 29; 1024 of 2048 x 768 59 / 20 / [29].
     double outputs = 0;
-    for (int m = 0; m < members; m++) outputs += (double)batch * grp.d[m];
-    if (wgs > (1ll << 30) || outputs < (narrow ? 830e3 * slim_rounds : 1080e3 * wide_rounds)) return false;
-    const int cols = columns(narrow ? 64 : 128);
-    const dim3 grid((unsigned)wgs);
+    for (int m = 0; m < members; m++) outputs += (double)batch * d[epilogue == Q8Epilogue::SwiGlu ? 0 : m];
+    if ((narrow ? slim : wide) > (1ll << 30) || outputs < (narrow ? 830e3 * slim_rounds : 1080e3 * wide_rounds)) return 0;
+    return narrow ? 64 : 128;
+}
+
+int q8_tile_rows(int launch, int batch, int n, int d, int d_kv) {
+    const Q8Epilogue epilogue[] = {Q8Epilogue::Store, Q8Epilogue::Residual, Q8Epilogue::SwiGlu, Q8Epilogue::Rope};
+    const int ds[3] = {d, d_kv, d_kv};
+    return batch > Q8_GEMV_MAX_BATCH && use_mma() ? q8_gemm_tile(epilogue[launch], ds, batch, n) : 0;
+}
+
+bool launch_q8_gemm(Q8Epilogue epilogue, const Q8Group& grp, const float* x, const Q8Split& split, int batch, int n,
+                    const Q8Norm& nm, const Q8Resid& resid, const Q8Rope& rope, hipStream_t stream) {
+    const bool pre = epilogue != Q8Epilogue::Store;
+    if (pre)
+        for (int m = 0; m < members_of(epilogue); m++)
+            if (!grp.wt[m]) return false;
+    if (pre && !split.in && (!split.scratch || nm.weight)) return false;
+    if (epilogue == Q8Epilogue::SwiGlu && !split.out.planes) return false;
+    const int rows = q8_gemm_tile(epilogue, grp.d, batch, n);
+    if (rows == 0) return false;
+    const int cols = columns(epilogue, grp.d, rows);
+    const dim3 grid((unsigned)((batch + GEMM_BM - 1) / GEMM_BM * cols));
     const void* in = x;
     if (pre && split.in) {
         in = split.in;
@@ -554,7 +571,7 @@ bool launch_q8_gemm(Q8Epilogue epilogue, const Q8Group& grp, const float* x, con
             case Q8Epilogue::Rope: launch<Q8Epilogue::Rope, NT>(grid, stream, grp, in, batch, n, cols, nm, resid, split.out, rope); break;
         }
     };
-    if (narrow)
+    if (rows == 64)
         run(std::integral_constant<int, 4>{});
     else
         run(std::integral_constant<int, 8>{});

@@ -92,6 +92,17 @@ __device__ __forceinline__ void store_split(const Q8SplitOut& o, int row, int k,
 // What a large product does with its sums.
 enum class Q8Epilogue { Store, Residual, SwiGlu, Rope };
 
+// Compute units of the current device (256 where there is none).
+int device_cus();
+
+// Whether NITRO_Q8_MMA leaves the bf16 matrix-core kernels in use.
+bool use_mma();
+
+// Weight rows per workgroup (128 or 64) with which the large-batch kernel takes a
+// launch over matrices of d[] rows (wq, wk, wv; w1, w3 of d[0]; or one), 0 where it
+// does not.
+int q8_gemm_tile(Q8Epilogue epilogue, const int* d, int batch, int n);
+
 // The large-batch product (q8_gemm.hip): true if launched, false where the
 // shapes are not its own (the caller takes another kernel).
 bool launch_q8_gemm(Q8Epilogue epilogue, const Q8Group& grp, const float* x, const Q8Split& split, int batch, int n,

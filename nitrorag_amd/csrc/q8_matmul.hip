@@ -54,6 +54,27 @@
 #include "q8_group.hpp"
 
 namespace nitro {
+
+bool use_mma() {
+    static const bool on = [] {
+        const char* e = getenv("NITRO_Q8_MMA");
+        return !(e && e[0] == 'f');  // "f32": the fp32 matrix-core kernel (comparison runs)
+    }();
+    return on;
+}
+
+int device_cus() {
+    static int cus[64] = {};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+    if (cus[dev] == 0) {
+        int c = 0;
+        if (hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || c <= 0) c = 256;
+        cus[dev] = c;
+    }
+    return cus[dev];
+}
+
 namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -1443,14 +1464,6 @@ __global__ __launch_bounds__(64 * MMA_WAVES) void q8_mma_kernel(Q8Group grp, con
     }
 }
 
-bool use_mma() {
-    static const bool on = [] {
-        const char* e = getenv("NITRO_Q8_MMA");
-        return !(e && e[0] == 'f');  // "f32": the fp32 matrix-core kernel (comparison runs)
-    }();
-    return on;
-}
-
 // Row streaming pays off once a row has at least two 1024-k chunks (both k
 // halves busy).  Tiles are small (4R rows), so there are enough of them to
 // fill the GPU; past ROWDOT_MAX_GROUPS the workgroups loop over tiles.
@@ -1466,18 +1479,6 @@ int gemv_choice() {
         return e && e[0] == 's' ? 0 : e && e[0] == 'r' ? 1 : 2;
     }();
     return c;
-}
-
-int device_cus() {
-    static int cus[64] = {};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    if (cus[dev] == 0) {
-        int c = 0;
-        if (hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || c <= 0) c = 256;
-        cus[dev] = c;
-    }
-    return cus[dev];
 }
 
 // The flat kernel, if its activations and partial sums fit its LDS budget.

@@ -7,6 +7,8 @@ product out[b][i] = sum_k float(q[i][k]) * scale[i][k/32] * x[b][k] is fp32.
 """
 from __future__ import annotations
 
+import ctypes
+
 from . import _native as N
 from .attention import _dev, _stream_ptr
 
@@ -14,6 +16,16 @@ FULL_ROWS = 0    # matmul (src/model_q8.cpp:92-125)
 LAST_BLOCK = 1   # matmul_bulk (src/model_q8.cpp:382-420): only the last 32 columns count
 BLOCK = 32
 BLOCK_BYTES = 36
+# launches of tile_rows: q8_matmul, and a model's wo / w2, w1 + w3, wq + wk + wv
+MATMUL, RESIDUAL, SWIGLU, QKV = range(4)
+
+
+def tile_rows(batch: int, n: int, d: int, launch: int = MATMUL, d_kv: int = 0) -> int:
+    """Weight rows per workgroup (64 or 128) where the kernel for many rows takes a
+    full-row product, 0 where another kernel does (nitro_q8_tile_rows)."""
+    rows = ctypes.c_int32()
+    N.call("nitro_q8_tile_rows", launch, batch, n, d, d_kv, ctypes.byref(rows))
+    return rows.value
 
 
 def q8_matmul(w, x, out, semantics: int = FULL_ROWS, stream=None) -> None:

@@ -24,9 +24,10 @@ def gpu():
 
 @pytest.fixture(params=["x3", "mfma32", "valu"], autouse=True)
 def prefill_kernel(request, monkeypatch):
-    """Every prefill test runs on the three kernels: bf16 matrix cores with
-    three-part splits (default for hd <= 128), fp32 matrix cores
-    (NITRO_PREFILL_KERNEL=mfma32) and the VALU one (hd 256, or =valu)."""
+    """Every prefill test runs on the three kernels: bf16 matrix cores on exact
+    splits (the default at every head size), fp32 matrix cores
+    (NITRO_PREFILL_KERNEL=mfma32; head sizes other than 32, 64 and 128 then take
+    the VALU kernel) and the VALU one (=valu)."""
     monkeypatch.setenv("NITRO_PREFILL_KERNEL", request.param)
     return request.param
 
@@ -55,7 +56,7 @@ def run_prefill(k, v, layer, tables, start_pos, lens, q, kc, vc, H, Hkv, hd):
 
 
 # every paged prefill case of the reference's golden vectors (head sizes 16, 32, 64;
-# 16 runs the VALU kernel padded to 32 whichever kernel is asked for)
+# 16 runs padded to 32)
 @pytest.mark.parametrize("name", ["prefill_hd64", "prefill_gqa_hd32_l2", "prefix_hit_hd32",
                                   "prefill_fresh_hd16_l2", "prefill_continued_gqa", "prefix_hit_gqa_l2"])
 def test_prefill_matches_reference_golden(golden_attention, name):
@@ -137,8 +138,8 @@ CASES = {
     # tokens): the rest of the table is read from global memory
     "beyond_lds_table_hd64": (6, 2, 5, 40, 2, 2, 64, 1, 0, 33000, 33100),
     "beyond_lds_table_gqa_hd128": (7, 2, 5, 150, 2, 1, 128, 1, 0, 33000, 33100),
-    # head sizes other than 32/64/128/256 (multiples of 4): the VALU kernel with
-    # the head padded to the next kernel width and the extra columns masked
+    # head sizes between the kernels' widths (multiples of 4): padded to the next
+    # width, the extra columns masked; 96, a width of the default kernel only
     "hd16_gqa_4x2": (8, 3, 1, 90, 4, 2, 16, 1, 0, 0, 30),
     "hd48": (9, 3, 20, 140, 3, 3, 48, 2, 1, 0, 17),
     "hd80_gqa_6x2": (10, 2, 1, 120, 6, 2, 80, 1, 0, 5, 40),

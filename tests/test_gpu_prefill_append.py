@@ -81,9 +81,9 @@ FRESH = {
 }
 
 
-# fresh prompts and chunks after cached keys at head sizes 32, 64, 128 take the
-# one-launch form; head size 256 and padded sizes, and keys past the LDS copy of
-# the table (32k tokens) run the two launches behind the same call
+# fresh prompts and chunks after cached keys at head sizes 32, 64, 68..96 and 128
+# take the one-launch form; the other sizes, and keys past the LDS copy of the
+# table (32k tokens), run the two launches behind the same call
 @pytest.mark.parametrize("name,one_launch", [
     ("prompts_b8_12x64", True),
     ("fresh_gqa_8x2_hd128", True),
@@ -98,6 +98,8 @@ FRESH = {
     ("continued_gqa_16x4_hd64", True),
     ("chunk_256_after_512_hd64", True),
     ("chunk_256_after_256_hd128", True),
+    ("hd80_gqa_6x2", True),
+    ("hd96", True),
     ("mha_hd256", False),
     ("hd48", False),
     ("beyond_lds_table_hd64", False),
