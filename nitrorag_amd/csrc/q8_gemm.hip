@@ -353,7 +353,14 @@ __global__ __launch_bounds__(64 * GEMM_WAVES, GEMM_NT == 8 ? 2 : 3) void q8_gemm
         constexpr int COLS = SWIGLU ? GEMM_BN / 2 : GEMM_BN;
         float* const rows = reinterpret_cast<float*>(&sums[wave][0][0]);
         static_assert(16 * (COLS + 4) <= GEMM_MT * GEMM_NT * 256, "the outputs fit the wave's sums");
+        // Lanes read what other lanes of the wave wrote there, and write where others
+        // read: no access may pass another between them.
+        auto exchange = []() __attribute__((always_inline)) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        };
         auto write_split = [&]() __attribute__((always_inline)) {
+            exchange();
             if (b0 + 16 * m >= batch) return;  // wave-uniform
 #pragma unroll
             for (int j = 0; j < COLS / 32; j++) {
@@ -370,6 +377,7 @@ __global__ __launch_bounds__(64 * GEMM_WAVES, GEMM_NT == 8 ? 2 : 3) void q8_gemm
                 for (int i = 0; i < 3; i++) *reinterpret_cast<bf16x8*>(dst + 1024 * i) = p[i];
             }
         };
+        if constexpr (SWIGLU || EPI == Q8Epilogue::Residual) exchange();
         if constexpr (SWIGLU) {
             // the first half of the tiles are w1's rows, the second the same rows of w3
 #pragma unroll
