@@ -1200,11 +1200,10 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
             m = mm;
         }
     }
-    const float inv = 1.0f / lsum;
     uint32_t nan_rows = 0;  // VP 3: of the wave's 16 rows, those with a NaN output
     if constexpr (VP == 3) {
         // NaN where an output is NaN (or infinite): 0 times it
-        f32x4 z = {inv * 0.0f, 0.f, 0.f, 0.f};
+        f32x4 z = {1.0f / lsum * 0.0f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int n = 0; n < NB; n++)
 #pragma unroll
@@ -1214,7 +1213,8 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
         const uint32_t half = (uint32_t)lanes | (uint32_t)(lanes >> 32);
         nan_rows = (half | half >> 16) & 0xffffu;
     }
-    if (row < qcount && !((nan_rows >> ql) & 1)) {
+    if (row < qcount && (VP == 2 || !((nan_rows >> ql) & 1))) {
+        const float inv = 1.0f / lsum;
         float* op = a.out + qrow * dim + (size_t)h * hd;
 #pragma unroll
         for (int n = 0; n < NB; n++)

@@ -29,7 +29,8 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 //  - weights: a block of the rows is converted to bf16 (exact) into LDS, shared
 //    by the waves; two buffers, one barrier per block.  A row's four 16-byte
 //    runs are swizzled by (row / 2) % 4, so that 8 lanes reading or writing
-//    consecutive rows hit distinct banks.
+//    consecutive rows hit distinct banks (no conflict cycles in wq/wk/wv and
+//    q8_matmul; 0.05 per LDS instruction in the others, from their epilogues).
 //  - per block and tile, three products (lo, mid, hi parts) from zero give
 //    sum_k q*x, which is scaled into the accumulators by the lane's own weight
 //    row's scale.  Every GEMM_FLUSH blocks the accumulators are added to sums in
@@ -40,9 +41,11 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // Bound by the matrix cores and, at n = 768, by the first and last blocks of a
 // tile: w1/w3 of 5520 rows at 768 x 2048 370 -> 117 us with hb written split
 // (0.89 PFLOP/s of bf16 products, three per multiply), wq/wk/wv 216 -> 89, wo
-// 99 -> 40; 1600 rows at 4096 x 11008 are at 46% of the matrix cores' cycles (a
-// plain 8192^3 bf16 product reaches 50%).  Prompts of 8 users, 110M-parameter
-// shapes: 11.96 -> 4.6 ms; q8_matmul of 1024 rows, 4096 x 11008, three products: 5.18 -> 1.10 ms.
+// 99 -> 39, w2 75 us.  The matrix cores are busy in 45% of the CUs' cycles in
+// w1/w3, 36% in wq/wk/wv, wo and w2, 37 and 29% in q8_matmul of 1024 rows at 4096 x
+// 11008 (w1, w2), where a plain 8192^3 bf16 product has 73%.  Prompts of 8 users,
+// 110M-parameter shapes: 11.96 -> 4.5 ms; q8_matmul of 1024 rows, 4096 x 11008,
+// three products: 5.18 -> 1.08 ms.
 constexpr int GEMM_WAVES = 4;
 constexpr int GEMM_BM = 32 * GEMM_WAVES;
 constexpr int GEMM_MT = 2;            // 16-row batch tiles per wave

@@ -1638,6 +1638,15 @@ hipError_t launch_q8_tile(const void* w, void* tiled, int d, int n, hipStream_t 
     return hipGetLastError();
 }
 
+// Split form is read at 6 bytes a value where floats are 4, every 16 weight rows
+// anew (a tile of up to 8 rows reads half the lines), and saves its readers the
+// split and the norm.  It is taken at every size that fits: whole decode steps with
+// floats instead, in the same process and buffers, took from
+//   5..8 rows    1.03-1.05x (768 wide) .. 1.07-1.11x (2048) .. 1.13-1.14x (4096)
+//   12, 16       1.08, 1.10            .. 1.11, 1.16        .. 1.06, 1.10
+//   17, 32, 48   1.12, 1.11, 1.13      .. 1.19, 1.22, 1.29  .. 1.02, 1.08, 1.08
+// of the time; the least of 6 widths and 19 row counts were 9 and 10 rows of 3072
+// wide layers (0.987, 0.991) and 25 of 4096 (0.996).
 bool q8_split_usable(size_t rows, size_t dim, size_t hidden) {
     const size_t wide = std::max(dim, hidden);
     return use_mma() && rows > (size_t)Q8_GEMV_MAX_BATCH && q8_split_bytes(rows, wide) < (1ull << 32) &&
