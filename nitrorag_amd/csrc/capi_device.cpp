@@ -884,28 +884,25 @@ int nitro_prefill_batch_upload(nitro_kvpool* pool, const int32_t* tables, const 
         const size_t nt = (size_t)batch * max_pages;
         const size_t n_work = items.size() * 2, n_wide = wide.size() * 2;
         p.tables.reserve(nt);
-        p.d_start.reserve(batch);
-        p.d_len.reserve(batch);
-        p.d_row_off.reserve(batch);
+        p.seqs.reserve(batch);
         p.slots.reserve(total);
         p.row_pos.reserve(total);
         p.work.reserve(n_work);
         p.work_wide.reserve(n_wide);
         hipStream_t s = as_stream(stream);
         Staging& st = pool->prefill_staging;
-        st.acquire(nt + 3 * (size_t)batch + 2 * (size_t)total + n_work + n_wide, 8);
+        st.acquire(nt + 4 * (size_t)batch + 2 * (size_t)total + n_work + n_wide, 6);
         int32_t* h_tables = st.part(p.tables.ptr, nt);
-        int32_t* h_start = st.part(p.d_start.ptr, batch);
-        int32_t* h_len = st.part(p.d_len.ptr, batch);
-        int32_t* h_off = st.part(p.d_row_off.ptr, batch);
+        int32_t* h_seqs = st.part(&p.seqs.ptr->start_pos, 4 * (size_t)batch);
         int32_t* h_slots = st.part(p.slots.ptr, total);
         int32_t* h_row_pos = st.part(p.row_pos.ptr, total);
         int32_t* h_work = st.part(p.work.ptr, n_work);
         int32_t* h_wide = st.part(p.work_wide.ptr, n_wide);
         std::memcpy(h_tables, tables, nt * sizeof(int32_t));
-        std::memcpy(h_start, start_pos, batch * sizeof(int32_t));
-        std::memcpy(h_len, num_tokens, batch * sizeof(int32_t));
-        std::memcpy(h_off, row_off.data(), batch * sizeof(int32_t));
+        for (int b = 0; b < batch; b++) {
+            const PrefillSeq seq{start_pos[b], num_tokens[b], row_off[b], 0};
+            std::memcpy(h_seqs + 4 * (size_t)b, &seq, sizeof(seq));
+        }
         for (int b = 0; b < batch; b++)
             for (int t = 0; t < num_tokens[b]; t++) {
                 const int pos = start_pos[b] + t;
@@ -972,9 +969,7 @@ static PrefillLaunch prefill_args(nitro_kvpool* pool, int32_t layer, const float
     a.k_pool = pool->k;
     a.v_pool = pool->v;
     a.tables = p.tables.ptr;
-    a.start_pos = p.d_start.ptr;
-    a.num_tokens = p.d_len.ptr;
-    a.row_off = p.d_row_off.ptr;
+    a.seqs = p.seqs.ptr;
     a.work = p.work.ptr;
     a.bad_pages = pool->bad_pages.ptr;
     a.page_stride = pool->page_stride();

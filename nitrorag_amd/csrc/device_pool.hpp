@@ -63,7 +63,7 @@ struct DeviceBuffer {
 // The arrays of one upload: array p is words[p] words from word 4 * first[p] of
 // pinned host memory (each starts on 16 bytes), bound for dst[p].
 struct UploadParts {
-    static constexpr int MAX = 8;
+    static constexpr int MAX = 6;
     int32_t* dst[MAX];
     size_t words[MAX], first[MAX];
     int count;
@@ -192,10 +192,18 @@ struct DecodeBatch {
     uint64_t launches = 0, prefix_launches = 0;
 };
 
+// What a prefill kernel needs to know of a sequence: one 16-byte load (three
+// arrays cost a launch three cache lines: 406.6 us for 12 launches over 8 prompts,
+// 402.3 so).
+struct PrefillSeq {
+    int32_t start_pos, num_tokens, row_off, unused;
+};
+
 struct PrefillBatch {
     int32_t batch = 0, max_pages = 0, total_rows = 0, max_tokens = 0;
     std::vector<int32_t> start_pos, num_tokens, row_off;
-    DeviceBuffer<int32_t> tables, d_start, d_len, d_row_off;
+    DeviceBuffer<int32_t> tables;
+    DeviceBuffer<PrefillSeq> seqs;
     DeviceBuffer<int32_t> slots;      // per packed row: page*16 + row-in-page
     DeviceBuffer<int32_t> row_pos;    // per packed row: its position in the sequence
     DeviceBuffer<int32_t> work;       // per work item: (seq, first query) pairs
@@ -405,9 +413,8 @@ hipError_t launch_embed_rows(const float* table, const int32_t* tokens, float* x
                              int vocab, int32_t* bad_tokens, float* ss, const Q8SplitOut& split, hipStream_t stream);
 hipError_t launch_add_rmsnorm(float* x, const float* delta, const float* weight, float* out, int rows,
                               int dim, hipStream_t stream);
-hipError_t launch_gather_last_rows(const float* x, const float* ffn, const int32_t* row_off,
-                                  const int32_t* len, float* last, int chunks, int dim,
-                                  hipStream_t stream);
+hipError_t launch_gather_last_rows(const float* x, const float* ffn, const PrefillSeq* seqs, float* last,
+                                  int chunks, int dim, hipStream_t stream);
 hipError_t launch_swiglu(float* hb, const float* hb2, size_t n, hipStream_t stream);
 hipError_t launch_f32_matmul(const float* w, const float* x, float* out, int batch, int n, int d,
                              hipStream_t stream);
@@ -450,9 +457,7 @@ struct PrefillLaunch {
     int32_t append_mixed;  // appending form: some chunk starts after cached keys (read from the pool)
     int32_t max_pos;  // largest position of the batch
     const int32_t* tables;
-    const int32_t* start_pos;
-    const int32_t* num_tokens;
-    const int32_t* row_off;
+    const PrefillSeq* seqs;
     const int32_t* work;  // pairs (seq, first query row of the chunk)
     int32_t* bad_pages;
     int64_t page_stride, layer_off;

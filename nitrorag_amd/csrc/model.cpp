@@ -444,8 +444,7 @@ int nitro_forward_prefill(nitro_model* m, nitro_kvpool* pool, const int32_t* tok
                     ERR_INVALID_ARGUMENT, nitro_last_error());
         });
         // Each chunk's last token: rms_norm; logits = wcls . x (:553-555)
-        hip_check(launch_gather_last_rows(m->x.ptr, nullptr, p.d_row_off.ptr, p.d_len.ptr, m->last.ptr,
-                                          p.batch, m->dim, s),
+        hip_check(launch_gather_last_rows(m->x.ptr, nullptr, p.seqs.ptr, m->last.ptr, p.batch, m->dim, s),
                   "gather launch");
         hip_check(launch_add_rmsnorm(m->last.ptr, nullptr, m->f32(m->o_rms_final), m->last.ptr, p.batch,
                                      m->dim, s),

@@ -97,14 +97,13 @@ __global__ __launch_bounds__(ROW_THREADS) void add_rmsnorm_kernel(float* x,
     for (int i = threadIdx.x; i < dim; i += ROW_THREADS) orow[i] = weight[i] * (inv * xr[i]);
 }
 
-// last[b] = x[r] (+ ffn[r] when given) for the last row r = row_off[b] + len[b] - 1 of chunk b.
+// last[b] = x[r] (+ ffn[r] when given) for the last row r of chunk b.
 __global__ __launch_bounds__(ROW_THREADS) void gather_last_rows_kernel(const float* __restrict__ x,
                                                                        const float* __restrict__ ffn,
-                                                                       const int32_t* __restrict__ row_off,
-                                                                       const int32_t* __restrict__ len,
+                                                                       const PrefillSeq* __restrict__ seqs,
                                                                        float* __restrict__ last, int dim) {
     const int b = blockIdx.x;
-    const size_t r = (size_t)(row_off[b] + len[b] - 1);
+    const size_t r = (size_t)(seqs[b].row_off + seqs[b].num_tokens - 1);
     for (int i = threadIdx.x; i < dim; i += ROW_THREADS)
         last[(size_t)b * dim + i] = ffn ? x[r * dim + i] + ffn[r * dim + i] : x[r * dim + i];
 }
@@ -472,11 +471,10 @@ hipError_t launch_add_rmsnorm(float* x, const float* delta, const float* weight,
     return hipGetLastError();
 }
 
-hipError_t launch_gather_last_rows(const float* x, const float* ffn, const int32_t* row_off,
-                                  const int32_t* len, float* last, int chunks, int dim,
-                                  hipStream_t stream) {
+hipError_t launch_gather_last_rows(const float* x, const float* ffn, const PrefillSeq* seqs, float* last,
+                                  int chunks, int dim, hipStream_t stream) {
     hipLaunchKernelGGL(gather_last_rows_kernel, dim3(chunks), dim3(ROW_THREADS), 0, stream, x, ffn,
-                       row_off, len, last, dim);
+                       seqs, last, dim);
     return hipGetLastError();
 }
 

@@ -105,8 +105,9 @@ __global__ __launch_bounds__(THREADS) void paged_attn_prefill_kernel(PrefillLaun
     const int seq = a.work[2 * item];
     const int q0 = a.work[2 * item + 1];
     const int kv_h = h / a.kv_mul;
-    const int start = a.start_pos[seq];
-    const int qcount = min(BM, a.num_tokens[seq] - q0);
+    const PrefillSeq sq = a.seqs[seq];
+    const int start = sq.start_pos;
+    const int qcount = min(BM, sq.num_tokens - q0);
     const int row = threadIdx.x >> 2;
     const int c = threadIdx.x & 3;
     const int last_pos = start + q0 + qcount - 1;
@@ -114,7 +115,7 @@ __global__ __launch_bounds__(THREADS) void paged_attn_prefill_kernel(PrefillLaun
     const int32_t* trow = a.tables + (size_t)seq * a.max_pages;
     const int n_tiles = last_pos / BN + 1;
     const size_t dim = (size_t)a.n_heads * hd;
-    const size_t qrow = (size_t)(a.row_off[seq] + q0 + min(row, qcount - 1));
+    const size_t qrow = (size_t)(sq.row_off + q0 + min(row, qcount - 1));
 
     float4 qv[SLOTS];
     {
@@ -327,8 +328,9 @@ __global__ __launch_bounds__(64 * QT * KSPLIT) void paged_attn_prefill_mfma_kern
     const int seq = a.work[2 * item];
     const int q0 = a.work[2 * item + 1];
     const int kv_h = h / a.kv_mul;
-    const int start = a.start_pos[seq];
-    const int qcount = min(BM, a.num_tokens[seq] - q0);  // queries of the work item
+    const PrefillSeq sq = a.seqs[seq];
+    const int start = sq.start_pos;
+    const int qcount = min(BM, sq.num_tokens - q0);  // queries of the work item
     if (sub0 * 16 >= qcount) return;  // no query in this part (uniform)
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -344,7 +346,7 @@ __global__ __launch_bounds__(64 * QT * KSPLIT) void paged_attn_prefill_mfma_kern
     const int32_t* trow = a.tables + (size_t)seq * a.max_pages;
     const int n_tiles = last_pos / BNM + 1;
     const size_t dim = (size_t)a.n_heads * HD;
-    const size_t qrow = (size_t)(a.row_off[seq] + q0 + min(row, qcount - 1));
+    const size_t qrow = (size_t)(sq.row_off + q0 + min(row, qcount - 1));
 
     // The workgroup's block-table slice -> LDS (read once instead of per tile).
     const int n_pages = min((last_pos >> 4) + 1, TABLE_LDS);
@@ -591,15 +593,16 @@ __device__ __forceinline__ void prefill_row_fp32(const PrefillLaunch& a, int at,
     asm volatile("" ::: "memory");
     const int h = blockIdx.x % a.n_heads, item = blockIdx.x / a.n_heads;
     const int seq = a.work[2 * item], row = a.work[2 * item + 1] + at;
-    const int start = a.start_pos[seq], pos = start + row;
+    const PrefillSeq sq = a.seqs[seq];
+    const int start = sq.start_pos, pos = start + row;
     const int32_t* trow = a.tables + (size_t)seq * a.max_pages;
     const size_t col0 = (size_t)(h / a.kv_mul) * hd;
-    const size_t qat = (size_t)(a.row_off[seq] + row) * a.n_heads * hd + (size_t)h * hd;
+    const size_t qat = (size_t)(sq.row_off + row) * a.n_heads * hd + (size_t)h * hd;
     // a key's row of the head; null on a page outside the pool (a row of zeros)
     auto row_of = [&](const float* pool, const float* fresh, int key) -> const float* {
         const int page = trow[key >> 4];
         if ((unsigned)page >= (unsigned)a.num_pages) return nullptr;
-        if (APPEND && key >= start) return fresh + (size_t)(a.row_off[seq] + key - start) * a.kv_dim + col0;
+        if (APPEND && key >= start) return fresh + (size_t)(sq.row_off + key - start) * a.kv_dim + col0;
         return pool + a.layer_off + (size_t)page * a.page_stride + (size_t)(key & 15) * a.kv_dim + col0;
     };
     float m = -INFINITY, l = 0.0f, o[COLS] = {};
@@ -753,8 +756,9 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
     const int seq = a.work[2 * item];
     const int q0 = a.work[2 * item + 1];
     const int kv_h = h / a.kv_mul;
-    const int start = a.start_pos[seq];
-    const int qcount = min(16 * QT, a.num_tokens[seq] - q0);
+    const PrefillSeq sq = a.seqs[seq];
+    const int start = sq.start_pos;
+    const int qcount = min(16 * QT, sq.num_tokens - q0);
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int qs = wave % QT;
@@ -769,7 +773,7 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
     const int32_t* trow = a.tables + (size_t)seq * a.max_pages;
     const int n_tiles = last_pos / BNM + 1;
     const size_t dim = (size_t)a.n_heads * hd;
-    const size_t qrow = (size_t)(a.row_off[seq] + q0 + min(row, qcount - 1));
+    const size_t qrow = (size_t)(sq.row_off + q0 + min(row, qcount - 1));
 
     // This lane's query at d = 32c + 8g .. +8, loaded before the table so the
     // two loads' latencies overlap; it is scaled and split into parts once
@@ -873,11 +877,11 @@ __global__ __launch_bounds__(64 * QT * KSPLIT, HD <= 64 ? 4 : 1) void paged_attn
     const bool appends = APPEND && h % a.kv_mul == 0;
     const int own_first = start + q0;
     const size_t rows16_b = 16 * vrow_b;
-    const size_t dk = APPEND ? (size_t)(reinterpret_cast<uintptr_t>(a.k_new + (size_t)a.row_off[seq] * a.kv_dim) -
+    const size_t dk = APPEND ? (size_t)(reinterpret_cast<uintptr_t>(a.k_new + (size_t)sq.row_off * a.kv_dim) -
                                         reinterpret_cast<uintptr_t>(a.k_pool + a.layer_off)) -
                                    (size_t)start * vrow_b
                              : 0;
-    const size_t dv = APPEND ? (size_t)(reinterpret_cast<uintptr_t>(a.v_new + (size_t)a.row_off[seq] * a.kv_dim) -
+    const size_t dv = APPEND ? (size_t)(reinterpret_cast<uintptr_t>(a.v_new + (size_t)sq.row_off * a.kv_dim) -
                                         reinterpret_cast<uintptr_t>(a.v_pool + a.layer_off)) -
                                    (size_t)start * vrow_b
                              : 0;
