@@ -97,13 +97,14 @@ __global__ __launch_bounds__(ROW_THREADS) void add_rmsnorm_kernel(float* x,
     for (int i = threadIdx.x; i < dim; i += ROW_THREADS) orow[i] = weight[i] * (inv * xr[i]);
 }
 
-// last[b] = x[r] (+ ffn[r] when given) for the last row r of chunk b.
+// last[b] = x[r] (+ ffn[r] when given) for the last row r of chunk b (of a chunk
+// without tokens: the row before its place, or row 0).
 __global__ __launch_bounds__(ROW_THREADS) void gather_last_rows_kernel(const float* __restrict__ x,
                                                                        const float* __restrict__ ffn,
                                                                        const PrefillSeq* __restrict__ seqs,
                                                                        float* __restrict__ last, int dim) {
     const int b = blockIdx.x;
-    const size_t r = (size_t)(seqs[b].row_off + seqs[b].num_tokens - 1);
+    const size_t r = (size_t)max(seqs[b].row_off + seqs[b].num_tokens - 1, 0);
     for (int i = threadIdx.x; i < dim; i += ROW_THREADS)
         last[(size_t)b * dim + i] = ffn ? x[r * dim + i] + ffn[r * dim + i] : x[r * dim + i];
 }

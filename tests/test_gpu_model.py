@@ -294,3 +294,29 @@ def test_forward_vs_oracle_on_synthetic_models(name):
         check_logits(got, want, f"{name} decode step {step}")
     torch.cuda.synchronize()
     assert pool.take_device_errors() == 0
+
+
+def test_prefill_with_chunks_of_no_tokens():
+    """Chunks without tokens, the first one too, beside others: theirs is a logits row
+    that means nothing, read from inside the activations, and the other chunks' are
+    those of a batch without them."""
+    import torch
+
+    import nitrorag_amd as na
+    from nitrorag_amd.model import FULL_ROWS, synthetic_model_file
+
+    say("prefill with empty chunks")
+    dim, hid, L, H, Hkv, V, S = MODELS["mha_hd64_l3"]
+    model = na.Model(synthetic_model_file(dim, hid, L, H, Hkv, V, S, seed=9))
+    lens = [0, 9, 0, 21]
+    tables = np.arange(8, dtype=np.int32).reshape(4, 2)
+    toks = np.random.default_rng(10).integers(0, V, sum(lens)).astype(np.int32)
+    outs = []
+    for rows in ([0, 1, 2, 3], [1, 3]):
+        pool = na.KVPool(8, L, model.kv_dim)
+        pool.upload_prefill_batch(tables[rows], [0] * len(rows), [lens[r] for r in rows])
+        outs.append(model.forward_prefill(pool, toks, semantics=FULL_ROWS).cpu().numpy())
+        torch.cuda.synchronize()
+        assert pool.take_device_errors() == 0
+    assert np.isfinite(outs[0]).all()
+    check_logits(outs[0][[1, 3]], outs[1], "beside empty chunks")
