@@ -35,13 +35,13 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 //    sum_k q*x, which is scaled into the accumulators by the lane's own weight
 //    row's scale.  Every GEMM_FLUSH blocks the accumulators are added to sums in
 //    LDS, so that no chain of fp32 adds is longer than GEMM_FLUSH + n / (32
-//    GEMM_FLUSH): error against 64 bits 0.79e-7 / 0.98e-7 / 1.2e-7 / 1.75e-7
+//    GEMM_FLUSH): error against 64 bits 0.78e-7 / 0.97e-7 / 1.2e-7 / 1.75e-7
 //    (2-norm) at n = 768 / 2048 / 4096 / 11008, as q8_mma_kernel's 0.80 / 0.97
 //    / 1.2 / 1.74, which adds eight waves' chains; one chain gave 1.0e-7 at 768.
 // Bound by the matrix cores and, at n = 768, by the first and last blocks of a
 // tile: w1/w3 of 5520 rows at 768 x 2048 370 -> 117 us with hb written split
 // (0.89 PFLOP/s of bf16 products, three per multiply), wq/wk/wv 216 -> 89, wo
-// 99 -> 39, w2 75 us.  The matrix cores are busy in 45% of the CUs' cycles in
+// 99 -> 39, w2 251 -> 78.  The matrix cores are busy in 45% of the CUs' cycles in
 // w1/w3, 36% in wq/wk/wv, wo and w2, 37 and 29% in q8_matmul of 1024 rows at 4096 x
 // 11008 (w1, w2), where a plain 8192^3 bf16 product has 73%.  Prompts of 8 users,
 // 110M-parameter shapes: 11.96 -> 4.5 ms; q8_matmul of 1024 rows, 4096 x 11008,
