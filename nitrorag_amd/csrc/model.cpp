@@ -32,9 +32,10 @@ struct nitro_model {
     size_t tiled_bytes = 0;
     size_t t_wq = 0, t_wk = 0, t_wv = 0, t_wo = 0, t_w1 = 0, t_w2 = 0, t_w3 = 0;
     DeviceBuffer<float> x, attn, q, last, ss;
-    DeviceBuffer<uint8_t> hb;      // SwiGLU's output: as floats, or in split form
-    DeviceBuffer<uint8_t> xsplit;  // x (times the next norm's weights) in split form
-    int max_rows = 0;              // of any forward
+    DeviceBuffer<float> hb;                // SwiGLU's output as floats (where hsplit does not hold them)
+    DeviceBuffer<uint8_t> xsplit, hsplit;  // x (times the next norm's weights) and that output in split form
+    int max_rows = 0;                      // of any forward
+    float* hb_floats() const { return hb.ptr ? hb.ptr : reinterpret_cast<float*>(hsplit.ptr); }
     DeviceBuffer<int32_t> tokens;
     Staging staging;
 
@@ -83,8 +84,10 @@ void ensure_tiled(nitro_model* m, hipStream_t s) {
 }
 
 // Room for a forward of `rows` rows.  A model that has run no full-row products of
-// more than 4 rows holds nothing in split form; one that has holds hb once, in the
-// larger of its two forms, for as many rows as any forward had.
+// more than 4 rows holds nothing in split form; one that has holds it for as many
+// rows as any forward had, and that memory serves SwiGLU's output as floats too
+// unless those have a buffer already.  Only a forward of more rows than any before
+// moves a buffer that exists (a captured forward holds their addresses).
 void reserve_rows(nitro_model* m, int rows, bool last_block) {
     m->max_rows = std::max(m->max_rows, rows);
     const size_t r = (size_t)m->max_rows;
@@ -93,16 +96,14 @@ void reserve_rows(nitro_model* m, int rows, bool last_block) {
     m->ss.reserve(r * (size_t)((m->dim + 15) / 16));
     m->q.reserve(r * m->dim);
     m->tokens.reserve(r);
-    size_t hb_bytes = r * m->hidden * sizeof(float);
     if (m->tiled || (!last_block && rows > Q8_GEMV_MAX_BATCH)) {
         const size_t sr = q8_split_usable(r, m->dim, m->hidden) ? r : (size_t)rows;
         if (q8_split_usable(sr, m->dim, m->hidden)) {
-            if (!m->xsplit.ptr) m->hb.reset();  // its one change of form: to the size, not to twice it
             m->xsplit.reserve(q8_split_bytes(sr, m->dim));
-            hb_bytes = std::max(hb_bytes, q8_split_bytes(sr, (size_t)std::max(m->dim, m->hidden)));
+            m->hsplit.reserve(q8_split_bytes(sr, (size_t)std::max(m->dim, m->hidden)));
         }
     }
-    m->hb.reserve(hb_bytes);
+    if (m->hb.ptr || m->hsplit.count < r * m->hidden * sizeof(float)) m->hb.reserve(r * m->hidden);
 }
 
 void check_model_pool(const nitro_model* m, const nitro_kvpool* pool) {
@@ -155,8 +156,8 @@ void layers(nitro_model* m, nitro_kvpool* pool, const int32_t* tokens, int rows,
     // the launch that made them.
     const bool use_split = !last && q8_split_usable(rows, dim, hid);
     char* const xs = reinterpret_cast<char*>(use_split ? m->xsplit.ptr : nullptr);
-    char* const hs = reinterpret_cast<char*>(use_split ? m->hb.ptr : nullptr);
-    float* const hb = reinterpret_cast<float*>(m->hb.ptr);
+    char* const hs = reinterpret_cast<char*>(use_split ? m->hsplit.ptr : nullptr);
+    float* const hb = m->hb_floats();
     auto x_out = [&](const float* next_norm) { return next_norm ? Q8SplitOut{xs, next_norm, dim / 32} : Q8SplitOut{}; };
     hip_check(launch_embed_rows(m->f32(m->o_emb), tokens, m->x.ptr, rows, dim, m->vocab, pool->bad_pages.ptr,
                                 m->ss.ptr, use_split ? x_out(m->f32(m->o_rms_att)) : Q8SplitOut{}, s),

@@ -1,23 +1,35 @@
-"""Device memory that a model's forwards take: one copy of the SwiGLU output, in the
-form the products read, and nothing in split form for a model that never runs
-full-row products of more than 4 rows."""
+"""Device memory that a model's forwards take: the SwiGLU output held once where
+every product reads one form of it, nothing in split form for a model that never runs
+full-row products of more than 4 rows, and no buffer moved by a forward of other
+semantics."""
 import numpy as np
 import pytest
+
+from nitrorag_amd.model import FULL_ROWS, LAST_BLOCK, synthetic_model_file
 
 pytestmark = pytest.mark.gpu
 
 DIM, HIDDEN, HEADS, VOCAB, SEQ = 256, 8192, 4, 64, 1024
 PROMPTS, TOKENS = 8, 1000
 ROWS = PROMPTS * TOKENS
+HB = 4 * ROWS * HIDDEN                              # SwiGLU's output as floats
+ROW_BUFFERS = 4 * ROWS * (3 * DIM + DIM // 16 + 1)  # x, attention, q, partial sums, tokens
+SPLIT = 6 * ROWS * (DIM + HIDDEN)                   # x and SwiGLU's output in split form
+WEIGHTS = 2 * (3 * HIDDEN + 4 * DIM) * DIM          # the tile layout, below 2 bytes a weight
+SLACK = 48 << 20                                    # allocation granules, kernels loaded on first use
 
 
-def test_forward_buffers():
+@pytest.mark.parametrize("order,most", [
+    ([LAST_BLOCK, LAST_BLOCK], [ROW_BUFFERS + HB] * 2),
+    ([FULL_ROWS, LAST_BLOCK, FULL_ROWS], [ROW_BUFFERS + SPLIT + WEIGHTS] * 3),
+    ([LAST_BLOCK, FULL_ROWS, LAST_BLOCK], [ROW_BUFFERS + HB] + [ROW_BUFFERS + HB + SPLIT + WEIGHTS] * 2),
+])
+def test_forward_buffers(order, most):
     import torch
 
     import nitrorag_amd as na
-    from nitrorag_amd.model import FULL_ROWS, LAST_BLOCK, synthetic_model_file
 
-    print("model buffers", flush=True)
+    print(f"model buffers, semantics {order}", flush=True)
     model = na.Model(synthetic_model_file(DIM, HIDDEN, 1, HEADS, HEADS, VOCAB, SEQ, seed=3))
     need = -(-TOKENS // 16)
     pages = torch.zeros((PROMPTS * need, 1, 16, model.kv_dim), device="cuda")
@@ -27,22 +39,14 @@ def test_forward_buffers():
     logits = torch.empty((PROMPTS, VOCAB), device="cuda")
     pool.upload_prefill_batch(tables, [0] * PROMPTS, [TOKENS] * PROMPTS)
     torch.cuda.synchronize()
-    free = [torch.cuda.mem_get_info()[0]]
-    outs = []
-    for semantics in (LAST_BLOCK, FULL_ROWS, LAST_BLOCK):
+    free, outs = torch.cuda.mem_get_info()[0], {}
+    for semantics, bound in zip(order, most):
         model.forward_prefill(pool, tokens, logits, semantics)
         torch.cuda.synchronize()
-        outs.append(logits.clone())
+        assert torch.isfinite(logits).all()
+        assert torch.equal(logits, outs.setdefault(semantics, logits.clone()))
         torch.cuda.synchronize()
-        free.append(torch.cuda.mem_get_info()[0])
-    assert torch.equal(outs[0], outs[2]) and torch.isfinite(outs[1]).all()
+        taken = free - torch.cuda.mem_get_info()[0]
+        print(f"semantics {semantics}: {taken} of {bound}", flush=True)
+        assert taken <= bound + SLACK
     assert pool.take_device_errors() == 0
-    taken = [free[0] - f for f in free[1:]]
-    floats = 4 * ROWS * (3 * DIM + DIM // 16 + HIDDEN)     # x, attention, q, partial sums, hb
-    split = 6 * ROWS * DIM + 2 * ROWS * HIDDEN             # x in split form; hb grows from 4 to 6 bytes a value
-    weights = 2 * (2 * HIDDEN + HIDDEN + 4 * DIM) * DIM    # the tile layout, below 2 bytes a weight
-    slack = 48 << 20                                       # allocation granules, kernels loaded on first use
-    print(f"taken {taken}, floats {floats}, split {split}", flush=True)
-    assert taken[0] <= floats + slack
-    assert taken[1] <= floats + split + weights + slack
-    assert taken[2] <= taken[1] + slack
